@@ -492,24 +492,73 @@ int sigma_assemble(hipStream_t s, const double* d_spec, const double* d_zz, cons
 }
 
 // ------------------------------------------------------------ QP Newton
-// Cubic spline of SIGMA/spline.f90:20-77 on one real table (nn points).
-__device__ void spline_dev(const double* xx, const double* yy, int nn, double yp1, double ypn,
-                           double* y2, double* uu)
+// The spline table of one QP state: xx(i) = x0 + step (i + 1), i < nn, the
+// inner points of the energy grid (spline_evaluate.f90 drops the end points
+// and uses them for the end slopes).
+struct SplineGrid {
+    double x0, step;
+    int nn;
+    __device__ __forceinline__ double x(int i) const { return x0 + step * (double)(i + 1); }
+};
+
+// Second derivatives of SIGMA/spline.f90:20-77 for the table f(0..nn+1) on
+// one wave: the end points f(0), f(nn + 1) give the end slopes, f + 1 is the
+// splined table.  On return y2(0..nn-1) holds the second derivatives.  c and
+// y2 first take the tridiagonal coefficients and right-hand sides, one row
+// per lane (all the divisions by grid steps in parallel); the two recurrences
+// then run in every lane on eight rows loaded ahead, so that a step waits for
+// one division (forward) or one fused multiply-add (backward), not for memory.
+__device__ void spline_wave(const SplineGrid& g, const double* f, double* c, double* y2)
 {
+    const int lane = threadIdx.x & 63, nn = g.nn;
     const double HUGEV = 1.0e10;
-    if (fabs(yp1) > HUGEV) {
-        y2[0] = 0.0;
-        uu[0] = 0.0;
-    } else {
-        y2[0] = -0.5;
-        uu[0] = (3.0 / (xx[1] - xx[0])) * ((yy[1] - yy[0]) / (xx[1] - xx[0]) - yp1);
+    const double* yy = f + 1;
+    const double yp1 = (f[1] - f[0]) / (g.x(0) - g.x(-1));
+    const double ypn = (f[nn + 1] - f[nn]) / (g.x(nn) - g.x(nn - 1));
+    for (int i = lane + 1; i < nn - 1; i += 64) {
+        const double xm = g.x(i - 1), x = g.x(i), xp = g.x(i + 1);
+        c[i] = (x - xm) / (xp - xm);
+        y2[i] = 6.0 * ((yy[i + 1] - yy[i]) / (xp - x) - (yy[i] - yy[i - 1]) / (x - xm)) / (xp - xm);
     }
-    for (int i = 1; i < nn - 1; ++i) {
-        double sig = (xx[i] - xx[i - 1]) / (xx[i + 1] - xx[i - 1]);
-        double p = sig * y2[i - 1] + 2.0;
-        y2[i] = (sig - 1.0) / p;
-        uu[i] = (6.0 * ((yy[i + 1] - yy[i]) / (xx[i + 1] - xx[i]) - (yy[i] - yy[i - 1]) / (xx[i] - xx[i - 1])) /
-                     (xx[i + 1] - xx[i - 1]) - sig * uu[i - 1]) / p;
+    __syncthreads();
+    constexpr int CH = 8;
+    double cc, uu;  // y2(i) = c(i) y2(i+1) + u(i)
+    if (fabs(yp1) > HUGEV) {
+        cc = 0.0;
+        uu = 0.0;
+    } else {
+        cc = -0.5;
+        uu = (3.0 / (g.x(1) - g.x(0))) * ((yy[1] - yy[0]) / (g.x(1) - g.x(0)) - yp1);
+    }
+    const double c0 = cc, u0 = uu;
+    for (int i0 = 1; i0 < nn - 1; i0 += CH) {
+        double sg[CH], r[CH];
+#pragma unroll
+        for (int k = 0; k < CH; ++k) {
+            const int i = min(i0 + k, nn - 2);
+            sg[k] = c[i];
+            r[k] = y2[i];
+        }
+#pragma unroll
+        for (int k = 0; k < CH; ++k) {
+            if (i0 + k >= nn - 1) break;
+            const double p = sg[k] * cc + 2.0;
+            cc = (sg[k] - 1.0) / p;
+            uu = (r[k] - sg[k] * uu) / p;
+            sg[k] = cc;
+            r[k] = uu;
+        }
+        if (lane < CH && i0 + lane < nn - 1) {
+            double cv = sg[0], uv = r[0];
+#pragma unroll
+            for (int k = 1; k < CH; ++k)
+                if (lane == k) {
+                    cv = sg[k];
+                    uv = r[k];
+                }
+            c[i0 + lane] = cv;
+            y2[i0 + lane] = uv;
+        }
     }
     double qn, un;
     if (ypn > HUGEV) {
@@ -517,96 +566,150 @@ __device__ void spline_dev(const double* xx, const double* yy, int nn, double yp
         un = 0.0;
     } else {
         qn = 0.5;
-        un = (3.0 / (xx[nn - 1] - xx[nn - 2])) * (ypn - (yy[nn - 1] - yy[nn - 2]) / (xx[nn - 1] - xx[nn - 2]));
+        un = (3.0 / (g.x(nn - 1) - g.x(nn - 2))) *
+             (ypn - (yy[nn - 1] - yy[nn - 2]) / (g.x(nn - 1) - g.x(nn - 2)));
     }
-    y2[nn - 1] = (un - qn * uu[nn - 2]) / (qn * y2[nn - 2] + 1.0);
-    for (int k = nn - 2; k >= 0; --k) y2[k] = y2[k] * y2[k + 1] + uu[k];
+    double v = (un - qn * uu) / (qn * cc + 1.0);
+    __syncthreads();
+    if (lane == 0) {
+        y2[nn - 1] = v;
+        c[0] = c0;
+        y2[0] = u0;
+    }
+    __syncthreads();
+    for (int i0 = nn - 2; i0 >= 0; i0 -= CH) {
+        double cv[CH], uv[CH];
+#pragma unroll
+        for (int k = 0; k < CH; ++k) {
+            const int i = max(i0 - k, 0);
+            cv[k] = c[i];
+            uv[k] = y2[i];
+        }
+#pragma unroll
+        for (int k = 0; k < CH; ++k) {
+            if (i0 - k < 0) break;
+            v = cv[k] * v + uv[k];
+            uv[k] = v;
+        }
+        if (lane < CH && i0 - lane >= 0) {
+            double o = uv[0];
+#pragma unroll
+            for (int k = 1; k < CH; ++k)
+                if (lane == k) o = uv[k];
+            y2[i0 - lane] = o;
+        }
+    }
+    __syncthreads();
 }
 
-// SIGMA/splint.f90:12-53.
-__device__ double splint_dev(const double* xx, const double* yy, const double* y2, int nn, double x0)
+// SIGMA/splint.f90:12-53 on the inner points.
+__device__ double splint_dev(const SplineGrid& g, const double* f, const double* y2, double x0)
 {
-    int klo = 1, khi = nn;
+    const double* yy = f + 1;
+    int klo = 1, khi = g.nn;
     while (khi - klo > 1) {
         int kk = (khi + klo) / 2;
-        if (xx[kk - 1] > x0) khi = kk; else klo = kk;
+        if (g.x(kk - 1) > x0) khi = kk; else klo = kk;
     }
-    double hh = xx[khi - 1] - xx[klo - 1];
-    double aa = (xx[khi - 1] - x0) / hh;
-    double bb = (x0 - xx[klo - 1]) / hh;
+    const double xl = g.x(klo - 1), xh = g.x(khi - 1);
+    double hh = xh - xl;
+    double aa = (xh - x0) / hh;
+    double bb = (x0 - xl) / hh;
     return aa * yy[klo - 1] + bb * yy[khi - 1] +
            ((aa * aa * aa - aa) * y2[klo - 1] + (bb * bb * bb - bb) * y2[khi - 1]) * (hh * hh) / 6.0;
 }
 
-// SIGMA/spline_evaluate.f90:13-51 for a real table.
-__device__ void spline_eval_dev(int nt, const double* xt, const double* ft, double x, double* fx,
-                                double* df, double* y2, double* uu)
+// SIGMA/spline_evaluate.f90:13-51 on a splined table: value at x and the
+// slope over +-0.01, the three points in lanes 0, 1 and 2 (all lanes return
+// them).
+__device__ __forceinline__ void spline_eval_wave(const SplineGrid& g, const double* f, const double* y2, double x,
+                                                 double* fx, double* df)
 {
-    const int nn = nt - 2;
-    double yp1 = (ft[1] - ft[0]) / (xt[1] - xt[0]);
-    double ypn = (ft[nt - 1] - ft[nt - 2]) / (xt[nt - 1] - xt[nt - 2]);
-    spline_dev(xt + 1, ft + 1, nn, yp1, ypn, y2, uu);
     const double DELTAX = 1.0e-2;
-    *fx = splint_dev(xt + 1, ft + 1, y2, nn, x);
-    double ym = splint_dev(xt + 1, ft + 1, y2, nn, x - DELTAX);
-    double yp = splint_dev(xt + 1, ft + 1, y2, nn, x + DELTAX);
-    *df = (yp - ym) / DELTAX * 0.5;
+    const int lane = threadIdx.x & 63;
+    const double at = lane == 1 ? x - DELTAX : lane == 2 ? x + DELTAX : x;
+    const double v = splint_dev(g, f, y2, at);
+    *fx = __shfl(v, 0);
+    *df = (__shfl(v, 2) - __shfl(v, 1)) / DELTAX * 0.5;
 }
 
-// One QP state per thread, SIGMA/printsigma.F90:97-128 with newtonr
+// One QP state per workgroup, SIGMA/printsigma.F90:97-128 with newtonr
 // (SIGMA/newtonr.f90:18-58, EN_ACC = 0.01 eV, 20 iterations).
 // in  (per state): [edft, en0, sigx, vxc]  at in[4*iq], then Sigma_c(nen) complex
 //                  at in[4*nqp + 2*nen*iq]
 // out (per state): [eqp, zfac, sigma0_re, sigma0_im, imsig, ierr]
-__global__ void qp_newton_kernel(int nqp, int nen, double deltae_ev, const double* in, double* out,
-                                 double* scratch)
+// The tables do not change during the root search, so each is splined once.
+// A serial chain of two divisions per grid point bounds the kernel; with the
+// tables in LDS (WIDE: two waves, one per table, up to QP_LDS_NEN points,
+// 48 KB) 64 states x 200 points take 41 us, against 1255 us for one thread
+// per state that splined the table again for every evaluation from global
+// memory.  Longer tables run on one wave in the global work arrays
+// (3 nen of the 5 nen doubles per state), one table after the other.
+constexpr int QP_LDS_NEN = 1024;
+template <bool WIDE>
+__global__ __launch_bounds__(WIDE ? 128 : 64) void qp_newton_kernel(int nqp, int nen, double deltae_ev,
+                                                                    const double* in, double* out, double* scratch)
 {
-    const int iq = blockIdx.x * blockDim.x + threadIdx.x;
-    if (iq >= nqp) return;
-    double* xt = scratch + (long)iq * 5 * nen;
-    double* ft = xt + nen;
-    double* it = ft + nen;
-    double* y2 = it + nen;
-    double* uu = y2 + nen;
+    extern __shared__ double qp_lds[];
+    const int iq = blockIdx.x;
+    const int tid = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    // table, coefficients, second derivatives of this wave
+    double* f = WIDE ? qp_lds + (long)wave * 3 * nen : scratch + (long)iq * 5 * nen;
+    double* c = f + nen;
+    double* y2 = c + nen;
     const double edft = in[4 * iq], en0 = in[4 * iq + 1], sigx = in[4 * iq + 2], vxc = in[4 * iq + 3];
     const double* sc = in + 4 * (long)nqp + 2 * (long)nen * iq;
-    for (int ii = 0; ii < nen; ++ii) {
-        xt[ii] = en0 - deltae_ev * 0.5 + deltae_ev / (double)(nen - 1) * (double)ii;
-        ft[ii] = sigx + sc[2 * ii] - vxc + edft - xt[ii];
-        it[ii] = sc[2 * ii + 1];
-    }
-    double e = en0, fx = 0.0, df = 0.0;
+    const SplineGrid g{en0 - deltae_ev * 0.5, deltae_ev / (double)(nen - 1), nen - 2};
+    for (int ii = tid; ii < nen; ii += 64)
+        f[ii] = wave == 0 ? sigx + sc[2 * ii] - vxc + edft - g.x(ii - 1) : sc[2 * ii + 1];
+    __syncthreads();
+    spline_wave(g, f, c, y2);
+    double e = en0, fx = 0.0, df = 0.0, s0 = 0.0, zf = 0.0, si = 0.0, xtmp;
     int ierr = 21;
-    for (int jj = 1; jj <= 20; ++jj) {
-        spline_eval_dev(nen, xt, ft, e, &fx, &df, y2, uu);
-        double dx = fx / df;
-        e = e - dx;
-        if (fabs(dx) < 0.01) {
-            spline_eval_dev(nen, xt, ft, e, &fx, &df, y2, uu);
-            ierr = 0;
-            break;
+    if (wave == 0) {
+        for (int jj = 1; jj <= 20; ++jj) {
+            spline_eval_wave(g, f, y2, e, &fx, &df);
+            const double dx = fx / df;
+            e = e - dx;
+            if (fabs(dx) < 0.01) {
+                ierr = 0;
+                break;
+            }
+        }
+        spline_eval_wave(g, f, y2, e, &s0, &zf);
+        spline_eval_wave(g, f, y2, edft, &s0, &xtmp);
+        s0 = s0 + vxc;
+        zf = -1.0 / zf;
+    }
+    if constexpr (!WIDE) {
+        __syncthreads();
+        for (int ii = tid; ii < nen; ii += 64) f[ii] = sc[2 * ii + 1];
+        __syncthreads();
+        spline_wave(g, f, c, y2);
+    }
+    if (wave == 0) {
+        si = splint_dev(g, WIDE ? f + 3 * nen : f, WIDE ? y2 + 3 * nen : y2, e);
+        if (tid == 0) {
+            double* o = out + 6 * (long)iq;
+            o[0] = e;
+            o[1] = zf;
+            o[2] = s0;
+            o[3] = 0.0;
+            o[4] = si;
+            o[5] = (double)ierr;
         }
     }
-    double s0, zf, xtmp, si;
-    spline_eval_dev(nen, xt, ft, e, &s0, &zf, y2, uu);
-    spline_eval_dev(nen, xt, ft, edft, &s0, &xtmp, y2, uu);
-    s0 = s0 + vxc;
-    zf = -1.0 / zf;
-    spline_eval_dev(nen, xt, it, e, &si, &xtmp, y2, uu);
-    double* o = out + 6 * (long)iq;
-    o[0] = e;
-    o[1] = zf;
-    o[2] = s0;
-    o[3] = 0.0;
-    o[4] = si;
-    o[5] = (double)ierr;
 }
 
 int qp_newton(hipStream_t s, int nqp, int nen, double deltae_ev, const double* d_in, double* d_out,
               double* d_scratch)
 {
-    hipLaunchKernelGGL(qp_newton_kernel, dim3((nqp + 63) / 64), dim3(64), 0, s, nqp, nen, deltae_ev,
-                       d_in, d_out, d_scratch);
+    if (nen <= QP_LDS_NEN)
+        hipLaunchKernelGGL(qp_newton_kernel<true>, dim3(nqp), dim3(128), sizeof(double) * 6 * nen, s, nqp, nen,
+                           deltae_ev, d_in, d_out, d_scratch);
+    else
+        hipLaunchKernelGGL(qp_newton_kernel<false>, dim3(nqp), dim3(64), 0, s, nqp, nen, deltae_ev, d_in, d_out,
+                           d_scratch);
     NGW_HIP(hipGetLastError());
     return NGW_OK;
 }
