@@ -80,10 +80,7 @@ __global__ __launch_bounds__(GNT) void gk1_kernel(const GOp* ops, const GStage* 
     const int nv = op.nv, N = nv * op.nvec;
     const double* sx = op.tda ? nullptr : op.sqrtr;
     auto red_store = [&](int row, int col, double val) {
-        int gm = m0 + row, gn = n0 + col;
-        double p = 0.0;
-        if (gm < op.nmu && gn < N) p = val * op.psi[gm + (long)(gn % nv) * op.ldp];
-        sm.red[row][col] = p;
+        sm.red[row][col] = val * op.psi[min(m0 + row, op.nmu - 1) + (long)((n0 + col) % nv) * op.ldp];
     };
     AccF64<GK1M, GK1N> acc;
     gemm_f64_tile<GK1M, GK1N>(ColMajorA{op.psi + (long)nv * op.ldp, op.ldp, op.nmu}, XprimeB{sg.x, sx, op.ld, nv, N},

@@ -43,6 +43,7 @@ struct XprimeBlockB {
         const long p = p0 + (long)v * nc;
         return {x + (long)b * ldx + p, s ? s + p : nullptr};
     }
+    __device__ Handle shift(const Handle& h, int c) const { return {h.x + c, h.s ? h.s + c : nullptr}; }
     __device__ void fetch(const Handle& h, int c, double (&r)[2]) const
     {
         r[0] = h.x[c];
@@ -73,10 +74,7 @@ __global__ __launch_bounds__(GNT) void blk_k1_kernel(ColMajorA al, XprimeBlockB 
     AccF64<BK1M, BK1N> acc;
     gemm_f64_tile<BK1M, BK1N>(al, bl, m0, n0, nc, acc, sm.ab);
     for_acc_f64<BK1M, BK1N>(acc, [&](int row, int col, double val) {
-        const int gm = m0 + row, gn = n0 + col;
-        double p = 0.0;
-        if (gm < nmu && gn < N) p = val * psiv[gm + (long)(gn % nv) * ldp];
-        sm.red[row][col] = p;
+        sm.red[row][col] = val * psiv[min(m0 + row, nmu - 1) + (long)((n0 + col) % nv) * ldp];
     });
     __syncthreads();
     const int nend = min(n0 + BK1N, N);
@@ -116,13 +114,22 @@ __global__ __launch_bounds__(GNT) void blk_k3_kernel(ColMajorAT al, WeightedPsiV
     const int N = nv * nvec;
     AccF64<BK3M, BK3N> acc;
     gemm_f64_tile<BK3M, BK3N>(al, bl, m0, n0, nmu, acc, sm);
-    for_acc_f64<BK3M, BK3N>(acc, [&](int row, int col, double val) {
-        const int c = m0 + row, j = n0 + col;
-        if (c < nc && j < N) {
-            const int b = j / nv, v = j - b * nv;
-            ep.apply(p0 + (long)v * nc + c, b, val);
-        }
-    });
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int c0 = m0 + (wave & 1) * (BK3M / 2) + (lane >> 4), j0 = n0 + (wave >> 1) * (BK3N / 2) + (lane & 15);
+#pragma unroll
+    for (int j = 0; j < BK3N / 32; ++j) {
+        const int col = j0 + 16 * j;
+        if (col >= N) continue;
+        const int b = col / nv;
+        const long base = p0 + (long)(col - b * nv) * nc;
+        // the terms of a column's elements are loaded before any is stored
+        OperatorEpilogue::Terms t[BK3M / 8];
+#pragma unroll
+        for (int r = 0; r < BK3M / 8; ++r) t[r] = ep.load(base + min(c0 + 4 * r, nc - 1), b);
+#pragma unroll
+        for (int r = 0; r < BK3M / 8; ++r)
+            if (c0 + 4 * r < nc) ep.store(base + c0 + 4 * r, b, ep.value(t[r], acc.v[r / 4][j][r % 4]));
+    }
 }
 
 }  // namespace

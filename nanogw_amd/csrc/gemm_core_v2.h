@@ -13,8 +13,6 @@
 
 #include "gemm_core_lowp.h"
 
-#include <type_traits>
-
 namespace ngw {
 
 // LDS row layout of a slab (four 16-byte chunks of k per row), chosen per
@@ -95,21 +93,6 @@ template <class T>
 __device__ __forceinline__ T gload(const void* p)
 {
     return *(const __attribute__((address_space(1))) T*)(p);
-}
-
-// Compile-time loop: f(std::integral_constant<int, 0>) ... f(<N - 1>).
-template <int I, int N, class F>
-__device__ __forceinline__ void static_for_impl(F&& f)
-{
-    if constexpr (I < N) {
-        f(std::integral_constant<int, I>{});
-        static_for_impl<I + 1, N>(f);
-    }
-}
-template <int N, class F>
-__device__ __forceinline__ void static_for(F&& f)
-{
-    static_for_impl<0, N>(f);
 }
 
 // Padding of the operands' k extent (a multiple of every slab depth).

@@ -8,16 +8,7 @@ namespace ngw {
 // Vector blocks of the polynomial evaluation are FP64, or FP32 for the
 // Clenshaw intermediates of the low-precision modes (flag set): the element
 // i of a block stored as float is ((const float*)p)[i].
-__device__ __forceinline__ double vload(const double* p, bool f32, long i)
-{
-    return f32 ? (double)reinterpret_cast<const float*>(p)[i] : p[i];
-}
-__device__ __forceinline__ void vstore(double* p, bool f32, long i, double v)
-{
-    if (f32) reinterpret_cast<float*>(p)[i] = (float)v;
-    else p[i] = v;
-}
-
+//
 // Stage flags: which vector blocks of a stage are stored as FP32.  ST_QW32:
 // the stage's input x is the polynomial's argument q (FP64), and the
 // low-precision x' pass also writes q as FP32 (LpOp::q32); ST_Q32: the
@@ -30,7 +21,7 @@ enum { ST_X32 = 1, ST_Y32 = 2, ST_O32 = 4, ST_QW32 = 8, ST_Q32 = 16 };
 //   r   = alpha hx + bx x(idx) + by y(idx) + gamma v0(idx)
 //                                                (one Horner or Clenshaw stage)
 //   out = acc(idx) + r                           (Lanczos w += p(H) q)
-// x, y and out (and acc, which is out) may be FP32 blocks (flags).
+// All blocks FP64 (the low-precision modes have their own epilogue).
 struct OperatorEpilogue {
     const double* x = nullptr; long ldx = 0;
     const double* d = nullptr;
@@ -41,25 +32,46 @@ struct OperatorEpilogue {
     double* out = nullptr; long ldo = 0;
     double bx = 0.0;
     const double* y = nullptr; long ldy = 0; double by = 0.0;
-    int flags = 0;
 
-    __device__ __forceinline__ void apply(long idx, int b, double Y) const
+    // Everything an element needs from memory.  A thread loads the terms of
+    // several elements before it stores the first result: through apply()
+    // alone each store would hold back the next element's loads (the compiler
+    // cannot tell that out overlaps none of them).
+    struct Terms {
+        double s, d, x, y, v, a;
+    };
+    __device__ __forceinline__ Terms load(long idx, int b) const
     {
-        double sv = s ? s[idx] : 1.0;
-        double hx = (beta * sv) * Y;
-        double xv = 0.0;
+        Terms t{1.0, 0.0, 0.0, 0.0, 0.0, 0.0};
+        if (s) t.s = s[idx];
         if (x) {
-            xv = vload(x, flags & ST_X32, idx + (long)b * ldx);
-            double xp = s ? sv * xv : xv;
-            hx = d[idx] * xp + hx;
+            t.x = x[idx + (long)b * ldx];
+            t.d = d[idx];
+        }
+        if (y) t.y = y[idx + (long)b * ldy];
+        if (v0) t.v = v0[idx + (long)b * ldv0];
+        if (acc) t.a = acc[idx + (long)b * ldacc];
+        return t;
+    }
+    __device__ __forceinline__ double value(const Terms& t, double Y) const
+    {
+        double hx = (beta * t.s) * Y;
+        if (x) {
+            double xp = s ? t.s * t.x : t.x;
+            hx = t.d * xp + hx;
         }
         double r = alpha * hx;
-        if (bx != 0.0) r = r + bx * xv;
-        if (y) r = r + by * vload(y, flags & ST_Y32, idx + (long)b * ldy);
-        if (v0) r = r + gamma * v0[idx + (long)b * ldv0];
-        if (acc) r = vload(acc, flags & ST_O32, idx + (long)b * ldacc) + r;
-        vstore(out, flags & ST_O32, idx + (long)b * ldo, r);
+        if (bx != 0.0) r = r + bx * t.x;
+        if (y) r = r + by * t.y;
+        if (v0) r = r + gamma * t.v;
+        if (acc) r = t.a + r;
+        return r;
     }
+    __device__ __forceinline__ void store(long idx, int b, double r) const
+    {
+        out[idx + (long)b * ldo] = r;
+    }
+    __device__ __forceinline__ void apply(long idx, int b, double Y) const { store(idx, b, value(load(idx, b), Y)); }
 };
 
 // One operator application on nvec device vectors (the matvec of
@@ -88,7 +100,6 @@ struct OperatorArgs {
         e.acc = acc; e.ldacc = ldacc;
         e.out = out; e.ldo = ldo;
         e.bx = bx; e.y = y; e.ldy = ldy; e.by = by;
-        e.flags = flags;
         return e;
     }
 };

@@ -1,6 +1,7 @@
 // Operand loaders of the FP64 ISDF operator GEMMs.  row(mn) returns a per-row
-// handle; fetch() issues the raw loads of element (mn, k) from clamped
-// addresses; combine() forms the element.
+// handle; shift() moves it by a lane's own k once per tile; fetch() issues the
+// raw loads of element (mn, k), k the same for every lane, so that k times a
+// leading dimension is scalar arithmetic; combine() forms the element.
 #pragma once
 
 #include "gemm_core_lowp.h"
@@ -14,6 +15,7 @@ struct ColMajorA {  // A(m, k) = a[m + k*ld]
     typedef const double* Handle;
     const double* a; long ld; int MN;
     __device__ Handle row(int m) const { return a + m; }
+    __device__ Handle shift(Handle h, int k) const { return h + (long)k * ld; }
     __device__ void fetch(Handle h, int k, double (&r)[1]) const { r[0] = h[(long)k * ld]; }
     __device__ double combine(const double (&r)[1]) const { return r[0]; }
 };
@@ -23,6 +25,7 @@ struct ColMajorB {  // B(k, n) = b[k + n*ld]
     typedef const double* Handle;
     const double* b; long ld; int MN;
     __device__ Handle row(int n) const { return b + (long)n * ld; }
+    __device__ Handle shift(Handle h, int k) const { return h + k; }
     __device__ void fetch(Handle h, int k, double (&r)[1]) const { r[0] = h[k]; }
     __device__ double combine(const double (&r)[1]) const { return r[0]; }
 };
@@ -32,6 +35,7 @@ struct ColMajorAT {  // A(m, k) = a[k + m*ld]
     typedef const double* Handle;
     const double* a; long ld; int MN;
     __device__ Handle row(int m) const { return a + (long)m * ld; }
+    __device__ Handle shift(Handle h, int k) const { return h + k; }
     __device__ void fetch(Handle h, int k, double (&r)[1]) const { r[0] = h[k]; }
     __device__ double combine(const double (&r)[1]) const { return r[0]; }
 };
@@ -44,6 +48,11 @@ struct XprimeB {  // x'(c, j = v + nv b) = s(v,c) x_b(v,c); s == null means 1 (T
     {
         int b = j / nv, v = j - b * nv;
         return {x + (long)b * ldx + v, s ? s + v : nullptr};
+    }
+    __device__ Handle shift(const Handle& h, int c) const
+    {
+        const long o = (long)c * nv;
+        return {h.x + o, h.s ? h.s + o : nullptr};
     }
     __device__ void fetch(const Handle& h, int c, double (&r)[2]) const
     {
@@ -63,6 +72,7 @@ struct WeightedPsiVB {  // W(mu, j = v + nv b) = PsiV(mu, v) u(mu, b)
         int b = j / nv, v = j - b * nv;
         return {psiv + (long)v * ldp, u + (long)b * ldu};
     }
+    __device__ Handle shift(const Handle& h, int k) const { return {h.pv + k, h.ub + k}; }
     __device__ void fetch(const Handle& h, int mu, double (&r)[2]) const
     {
         r[0] = h.pv[mu];
@@ -70,12 +80,27 @@ struct WeightedPsiVB {  // W(mu, j = v + nv b) = PsiV(mu, v) u(mu, b)
     }
     __device__ double combine(const double (&r)[2]) const { return r[0] * r[1]; }
 };
+struct SlotPairB {  // t(nu, b) = first + second K1 slot of vector b (see k1_direct_kernel)
+    static constexpr bool kContig = true;
+    static constexpr int NRAW = 2;
+    struct Handle { const double* p0; const double* p1; };
+    const double* tpart; long ldt; int MN;
+    __device__ Handle row(int b) const { return {tpart + (long)b * ldt, tpart + ((long)MN + b) * ldt}; }
+    __device__ Handle shift(const Handle& h, int k) const { return {h.p0 + k, h.p1 + k}; }
+    __device__ void fetch(const Handle& h, int nu, double (&r)[2]) const
+    {
+        r[0] = h.p0[nu];
+        r[1] = h.p1[nu];
+    }
+    __device__ double combine(const double (&r)[2]) const { return r[0] + r[1]; }
+};
 struct PairB {  // c_mn(nu) = Psi(nu, m_b) Psi(nu, n_b)  (P-vector build)
     static constexpr bool kContig = true;
     static constexpr int NRAW = 2;
     struct Handle { const double* pm; const double* pn; };
     const double* psi; long ld; const int* mband; const int* nband; int MN;
     __device__ Handle row(int b) const { return {psi + (long)mband[b] * ld, psi + (long)nband[b] * ld}; }
+    __device__ Handle shift(const Handle& h, int k) const { return {h.pm + k, h.pn + k}; }
     __device__ void fetch(const Handle& h, int nu, double (&r)[2]) const
     {
         r[0] = h.pm[nu];
