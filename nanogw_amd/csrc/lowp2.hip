@@ -727,16 +727,6 @@ __global__ __launch_bounds__(256) void wprep_kernel(const LpOp* ops, LpOp op1, c
 // 16-byte accesses of four consecutive elements (FP32 or FP64), widened to
 // or narrowed from FP64.
 __device__ __forceinline__ bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
-__device__ __forceinline__ void ld4(const float* p, double (&o)[4])
-{
-    const f32x4 v = *reinterpret_cast<const f32x4*>(p);
-    o[0] = (double)v.x; o[1] = (double)v.y; o[2] = (double)v.z; o[3] = (double)v.w;
-}
-__device__ __forceinline__ void ld4(const double* p, double (&o)[4])
-{
-    const double2 a = reinterpret_cast<const double2*>(p)[0], b = reinterpret_cast<const double2*>(p)[1];
-    o[0] = a.x; o[1] = a.y; o[2] = b.x; o[3] = b.y;
-}
 __device__ __forceinline__ void st4(float* p, const double (&r)[4])
 {
     *reinterpret_cast<f32x4*>(p) = f32x4{(float)r[0], (float)r[1], (float)r[2], (float)r[3]};
@@ -781,8 +771,6 @@ void k3v2_kernel(const LpOp* ops, LpOp op1, const LpStage* st, LpStage st1,
     const double beta = op.tda ? 2.0 : 4.0;
     const bool acc_on = sg.accumulate == 1 || (sg.accumulate == 2 && *op.kstep > 1);
     const bool use_q = op.q != nullptr && sg.gamma != 0.0;
-    // FP32 output stages read the first stage's FP32 copy of q
-    const float* q32 = (sg.flags & ST_Q32) && (sg.flags & ST_O32) ? op.q32 : nullptr;
     const long ncv = (long)nv * op.nc;
     const float* sigc = op.sig + nv;
     // element types of x, y, out fixed at compile time per flag combination
@@ -793,11 +781,17 @@ void k3v2_kernel(const LpOp* ops, LpOp op1, const LpStage* st, LpStage st1,
         const TX* xp = reinterpret_cast<const TX*>(sg.x);
         const TY* yp = reinterpret_cast<const TY*>(sg.y);
         TO* op_ = reinterpret_cast<TO*>(sg.out);
+        // FP32 output stages (ST_O32 comes with ST_Q32) read the first
+        // stage's FP32 copy of q
+        typedef std::conditional_t<sizeof(TO) == 4, float, double> TQ;
+        const TQ* qp;
+        if constexpr (sizeof(TO) == 4) qp = op.q32;
+        else qp = op.q;
         // four consecutive pairs icv = v..v+3 of one c share a b when nv is a
         // multiple of four (tiles start at multiples of four): then every
         // array is read and written with 16-byte accesses
         const bool vec = (nv & 3) == 0 && (op.ld & 3) == 0 && aligned16(xp) && aligned16(yp) && aligned16(op_) &&
-                         aligned16(use_q ? op.q : nullptr) && aligned16(q32) && aligned16(dp) &&
+                         aligned16(use_q ? qp : nullptr) && aligned16(dp) &&
                          (KIND != LP_F16 || aligned16(op.wsc)) && (ncv & 3) == 0;
         // The tile passes through LDS one accumulator fragment row at a time:
         // in pass q every wave writes its fragment row q (16 tile rows, so
@@ -810,6 +804,10 @@ void k3v2_kernel(const LpOp* ops, LpOp op1, const LpStage* st, LpStage st1,
         // so a pass frees its accumulators.  Pitch = BN + 16 floats: the 16
         // lanes of an accumulator row and the next row's 16 fall on disjoint
         // banks.
+        // All loads of a batch are issued before the first result is formed;
+        // ROOM: two waves per SIMD and at most 64 accumulator registers leave
+        // registers for twice the batch.
+        constexpr bool ROOM = KIND == LP_BF16X3;
         constexpr int FM = BM / 32, EPR = 32, PITCH = BN + 16, G = BN / 4, PER = EPR * G / GNT;
         static_assert(EPR * G % GNT == 0, "epilogue row blocks");
         static_assert(sizeof(sm) >= sizeof(float) * EPR * PITCH, "epilogue staging exceeds the slab LDS");
@@ -826,79 +824,121 @@ void k3v2_kernel(const LpOp* ops, LpOp op1, const LpStage* st, LpStage st1,
                     stg[hrow + 4 * (lane >> 4) + r][wn + 16 * jf + (lane & 15)] = acc.v[q][jf][r];
             __syncthreads();
             if (!vec) {
+                // a thread keeps one tile column (RS rows of the block per
+                // step) and has EB elements' loads in flight: consecutive
+                // lanes read consecutive pairs of one c
+                constexpr int RS = GNT / BN > 0 ? GNT / BN : 1, EB = ROOM ? 8 : 4;
+                static_assert(EPR / RS % EB == 0, "epilogue element batches");
+                const int col = (int)threadIdx.x % BN, j = n0 + col;
+                if ((int)threadIdx.x >= RS * BN || j >= N) return;
+                const int b = j / nv, v = j - b * nv, rl0 = (int)threadIdx.x / BN;
+                const long boff = (long)b * op.ld;
+                const TX* xb = xp + boff;
+                const TY* yb = yp + boff;
+                const TQ* qb = qp + (sizeof(TQ) == 4 ? (long)b * ncv : boff);
+                TO* ob = op_ + boff;
+                double wsj = 1.0;
+                if constexpr (KIND == LP_F16) wsj = (double)op.wsc[j] * F16_UNSCALE;
 #pragma unroll 1
-                for (int e = threadIdx.x; e < EPR * BN; e += GNT) {
-                    const int rl = e / BN, col = e - rl * BN;
-                    const int c = m0 + (rl < 16 ? 16 * q + rl : BM / 2 + 16 * q + rl - 16), j = n0 + col;
-                    if (c >= op.nc || j >= N) continue;
-                    const int b = j / nv, v = j - b * nv;
-                    const long idx = v + (long)c * nv, i = idx + (long)b * op.ld;
-                    double Y = (double)stg[rl][col] * (double)sigc[c];
-                    if constexpr (KIND == LP_F16) Y *= (double)op.wsc[j] * F16_UNSCALE;
-                    const float2 f = dp[idx];
-                    const double xv = (double)xp[i];
-                    const double hx = (double)f.x * xv + (beta * (double)f.y) * Y;
-                    double r = sg.alpha * hx + sg.bx * xv;
-                    if (yp) r = r + sg.by * (double)yp[i];
-                    if (use_q) r = r + sg.gamma * (q32 ? (double)q32[idx + (long)b * ncv] : op.q[i]);
-                    if (acc_on) r = (double)op_[i] + r;
-                    op_[i] = (TO)r;
+                for (int k0 = 0; k0 < EPR / RS; k0 += EB) {
+                    TX xv[EB];
+                    TY yv[EB];
+                    TQ qv[EB];
+                    TO av[EB];
+                    float sc[EB];
+                    float2 f[EB];
+                    // rows past the operand read its last row
+                    auto row = [&](int k) {
+                        const int rl = rl0 + RS * (k0 + k);
+                        return m0 + (rl < 16 ? 16 * q + rl : BM / 2 + 16 * q + rl - 16);
+                    };
+                    auto pair = [&](int k) { return v + min(row(k), op.nc - 1) * nv; };
+#pragma unroll
+                    for (int k = 0; k < EB; ++k) {
+                        sc[k] = sigc[min(row(k), op.nc - 1)];
+                        f[k] = dp[pair(k)];
+                        xv[k] = xb[pair(k)];
+                    }
+                    if (yp)
+#pragma unroll
+                        for (int k = 0; k < EB; ++k) yv[k] = yb[pair(k)];
+                    if (use_q)
+#pragma unroll
+                        for (int k = 0; k < EB; ++k) qv[k] = qb[pair(k)];
+                    if (acc_on)
+#pragma unroll
+                        for (int k = 0; k < EB; ++k) av[k] = ob[pair(k)];
+#pragma unroll
+                    for (int k = 0; k < EB; ++k) {
+                        double Y = (double)stg[rl0 + RS * (k0 + k)][col] * (double)sc[k];
+                        if constexpr (KIND == LP_F16) Y *= wsj;
+                        const double x1 = (double)xv[k];
+                        const double hx = (double)f[k].x * x1 + (beta * (double)f[k].y) * Y;
+                        double r = sg.alpha * hx + sg.bx * x1;
+                        if (yp) r = r + sg.by * (double)yv[k];
+                        if (use_q) r = r + sg.gamma * (double)qv[k];
+                        if (acc_on) r = (double)av[k] + r;
+                        if (row(k) < op.nc) ob[pair(k)] = (TO)r;
+                    }
                 }
                 return;
             }
-            // two groups in flight for the 128 x 192 tile (two waves per SIMD,
-            // with register room), one for 128 x 128 (three waves per SIMD)
-            // and for 128 x 256 (its accumulators leave no room)
-            constexpr int GUNROLL = BM * BN <= 128 * 128 || BM * BN > 128 * 192 ? 1 : 2;
-#pragma unroll GUNROLL
-            for (int k = 0; k < PER; ++k) {
-                const int e = threadIdx.x + GNT * k;
-                const int rl = e / G, cg = e - rl * G;
-                const int c = m0 + (rl < 16 ? 16 * q + rl : BM / 2 + 16 * q + rl - 16), j0 = n0 + 4 * cg;
-                if (c >= op.nc || j0 >= N) continue;
-                const f32x4 v4 = *reinterpret_cast<const f32x4*>(&stg[rl][4 * cg]);
-                const int b = j0 / nv, v0 = j0 - b * nv;
-                const long idx = v0 + (long)c * nv, i = idx + (long)b * op.ld;
-                // the stage's terms are added in the order of the element-wise
-                // form above, each array loaded just before it is needed
-                const double sc = (double)sigc[c];
-                const float va[4] = {v4.x, v4.y, v4.z, v4.w};
-                double res[4], xv[4], t4[4];
-                {
-                    float ws[4] = {1.0f, 1.0f, 1.0f, 1.0f};
-                    if constexpr (KIND == LP_F16) {
-                        const f32x4 w4 = *reinterpret_cast<const f32x4*>(op.wsc + j0);
-                        ws[0] = w4.x; ws[1] = w4.y; ws[2] = w4.z; ws[3] = w4.w;
-                    }
-                    ld4(xp + i, xv);
-                    const f32x4 d01 = *reinterpret_cast<const f32x4*>(dp + idx);
-                    const f32x4 d23 = *reinterpret_cast<const f32x4*>(dp + idx + 2);
-                    const float dd4[4] = {d01.x, d01.z, d23.x, d23.z}, ss4[4] = {d01.y, d01.w, d23.y, d23.w};
+            constexpr int GU = ROOM ? 2 : 1;  // groups with their loads in flight
+            static_assert(PER % GU == 0, "epilogue groups");
+#pragma unroll 1
+            for (int k0 = 0; k0 < PER; k0 += GU) {
+                typedef TX x4 __attribute__((ext_vector_type(4)));
+                typedef TY y4 __attribute__((ext_vector_type(4)));
+                typedef TO o4 __attribute__((ext_vector_type(4)));
+                typedef TQ q4 __attribute__((ext_vector_type(4)));
+                f32x4 ws[GU], d01[GU], d23[GU];
+                x4 xr[GU];
+                y4 yr[GU];
+                q4 qr[GU];
+                o4 ar[GU];
+                long ii[GU];
+                float sc[GU];
+                bool ok[GU];
+#pragma unroll
+                for (int g = 0; g < GU; ++g) {
+                    const int e = threadIdx.x + GNT * (k0 + g);
+                    const int rl = e / G, cg = e - rl * G;
+                    const int c = m0 + (rl < 16 ? 16 * q + rl : BM / 2 + 16 * q + rl - 16), j0 = n0 + 4 * cg;
+                    ok[g] = c < op.nc && j0 < N;
+                    const int cc = min(c, op.nc - 1), jc = min(j0, N - 4);  // loads past the end re-read the last
+                    const int b = jc / nv, idx = jc - b * nv + cc * nv;
+                    ii[g] = idx + (long)b * op.ld;
+                    sc[g] = sigc[cc];
+                    if constexpr (KIND == LP_F16) ws[g] = *reinterpret_cast<const f32x4*>(op.wsc + jc);
+                    xr[g] = *reinterpret_cast<const x4*>(xp + ii[g]);
+                    d01[g] = *reinterpret_cast<const f32x4*>(dp + idx);
+                    d23[g] = *reinterpret_cast<const f32x4*>(dp + idx + 2);
+                    if (yp) yr[g] = *reinterpret_cast<const y4*>(yp + ii[g]);
+                    if (use_q) qr[g] = *reinterpret_cast<const q4*>(qp + (sizeof(TQ) == 4 ? idx + (long)b * ncv : ii[g]));
+                    if (acc_on) ar[g] = *reinterpret_cast<const o4*>(op_ + ii[g]);
+                }
+#pragma unroll
+                for (int g = 0; g < GU; ++g) {
+                    const int e = threadIdx.x + GNT * (k0 + g);
+                    const int rl = e / G, cg = e - rl * G;
+                    const f32x4 v4 = *reinterpret_cast<const f32x4*>(&stg[rl][4 * cg]);
+                    // the terms are added in the order of the element-wise form
+                    const float dd4[4] = {d01[g].x, d01[g].z, d23[g].x, d23[g].z};
+                    const float ss4[4] = {d01[g].y, d01[g].w, d23[g].y, d23[g].w};
+                    double res[4];
 #pragma unroll
                     for (int u = 0; u < 4; ++u) {
-                        double Y = (double)va[u] * sc;
-                        if constexpr (KIND == LP_F16) Y *= (double)ws[u] * F16_UNSCALE;
-                        const double hx = (double)dd4[u] * xv[u] + (beta * (double)ss4[u]) * Y;
-                        res[u] = sg.alpha * hx + sg.bx * xv[u];
+                        const double x1 = (double)xr[g][u];
+                        double Y = (double)v4[u] * (double)sc[g];
+                        if constexpr (KIND == LP_F16) Y *= (double)ws[g][u] * F16_UNSCALE;
+                        const double hx = (double)dd4[u] * x1 + (beta * (double)ss4[u]) * Y;
+                        res[u] = sg.alpha * hx + sg.bx * x1;
+                        if (yp) res[u] = res[u] + sg.by * (double)yr[g][u];
+                        if (use_q) res[u] = res[u] + sg.gamma * (double)qr[g][u];
+                        if (acc_on) res[u] = (double)ar[g][u] + res[u];
                     }
+                    if (ok[g]) st4(op_ + ii[g], res);
                 }
-                if (yp) {
-                    ld4(yp + i, t4);
-#pragma unroll
-                    for (int u = 0; u < 4; ++u) res[u] = res[u] + sg.by * t4[u];
-                }
-                if (use_q) {
-                    if (q32) ld4(q32 + idx + (long)b * ncv, t4);
-                    else ld4(op.q + i, t4);
-#pragma unroll
-                    for (int u = 0; u < 4; ++u) res[u] = res[u] + sg.gamma * t4[u];
-                }
-                if (acc_on) {
-                    ld4(op_ + i, t4);
-#pragma unroll
-                    for (int u = 0; u < 4; ++u) res[u] = t4[u] + res[u];
-                }
-                st4(op_ + i, res);
             }
         });
     };
