@@ -578,13 +578,14 @@ __global__ __launch_bounds__(GNT) void k1v2_kernel(const LpOp* ops, LpOp op1, co
     constexpr int FM = BM / 32, FN = BN / 32;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int wm = (wave & 1) * (BM / 2), wn = (wave >> 1) * (BN / 2);
-    int vrow[FN];
-    bool cok[FN];
+    // (columns past N and rows past ldm1 hold zero sums; their Psi_v loads are
+    // clamped, not skipped: a branch around each load would make it wait for
+    // the one before)
+    const float* pcol[FN];
 #pragma unroll
     for (int j = 0; j < FN; ++j) {
-        const int gn = n0 + wn + 16 * j + (lane & 15);
-        cok[j] = gn < N;
-        vrow[j] = cok[j] ? gn % nv : 0;
+        const int gn = min(n0 + wn + 16 * j + (lane & 15), N - 1);
+        pcol[j] = op.psiv32 + (long)(gn % nv) * op.ldm1;
     }
 #pragma unroll
     for (int pass = 0; pass < BM / HALF; ++pass) {
@@ -593,27 +594,38 @@ __global__ __launch_bounds__(GNT) void k1v2_kernel(const LpOp* ops, LpOp op1, co
         for (int i = 0; i < FM; ++i) {
             const int row0 = wm + 16 * i + 4 * (lane >> 4);  // a fragment lies in one pass
             if (row0 < pass * HALF || row0 >= (pass + 1) * HALF) continue;
-            const int gm0 = m0 + row0;
+            const int gm0 = min(m0 + row0, op.ldm1 - 4);
+            f32x4 pv[FN];
+#pragma unroll
+            for (int j = 0; j < FN; ++j) pv[j] = *reinterpret_cast<const f32x4*>(pcol[j] + gm0);
 #pragma unroll
             for (int j = 0; j < FN; ++j) {
-                f32x4 pv = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-                if (cok[j] && gm0 < op.ldm1)
-                    pv = *reinterpret_cast<const f32x4*>(op.psiv32 + (long)vrow[j] * op.ldm1 + gm0);
                 const int col = wn + 16 * j + (lane & 15);
 #pragma unroll
-                for (int r = 0; r < 4; ++r) sm.red[row0 + r - pass * HALF][col] = acc.v[i][j][r] * pv[r];
+                for (int r = 0; r < 4; ++r) sm.red[row0 + r - pass * HALF][col] = acc.v[i][j][r] * pv[j][r];
             }
         }
         __syncthreads();
         for (int e = threadIdx.x; e < HALF * nbt; e += GNT) {
             int row = e % HALF, b = b_lo + e / HALF;
             int c0 = max(n0, b * nv) - n0, c1 = min(nend, (b + 1) * nv) - n0;
+            double sc = 1.0;
+            if constexpr (KIND == LP_F16) sc = (double)op.xsc[b] * (double)(1.0f / F16_VEC) * (double)(1.0f / F16_OPS);
+            // in column order, eight LDS reads in flight
             float sum = 0.0f;
-            for (int cc = c0; cc < c1; ++cc) sum += sm.red[row][cc];
+            int cc = c0;
+            for (; cc + 8 <= c1; cc += 8) {
+                float w[8];
+#pragma unroll
+                for (int k = 0; k < 8; ++k) w[k] = sm.red[row][cc + k];
+#pragma unroll
+                for (int k = 0; k < 8; ++k) sum += w[k];
+            }
+            for (; cc < c1; ++cc) sum += sm.red[row][cc];
             int gm = m0 + pass * HALF + row;
             int slot = tn - (b * nv) / BN;
             double t = (double)sum;
-            if constexpr (KIND == LP_F16) t *= (double)op.xsc[b] * (double)(1.0f / F16_VEC) * (double)(1.0f / F16_OPS);
+            if constexpr (KIND == LP_F16) t *= sc;
             if (gm < op.nmu) op.tpart[((long)slot * op.nvec + b) * op.nmu + gm] = t;
         }
     }
