@@ -21,6 +21,8 @@
 
 namespace ngw {
 
+static int tiles(long m, int bm, long n, int bn) { return (int)((m + bm - 1) / bm * ((n + bn - 1) / bn)); }
+
 // ---------------------------------------------------------------- plain GEMMs
 template <class AL, class BL>
 __global__ __launch_bounds__(GNT) void gemm_plain_kernel(AL al, BL bl, int m, int n, int k, double alpha,
@@ -55,6 +57,68 @@ int gemm_f64_tn(hipStream_t s, int m, int n, int k, double alpha, const double* 
     int mt = (m + 127) / 128, nt = (n + 127) / 128;
     hipLaunchKernelGGL((gemm_plain_kernel<ColMajorAT, ColMajorB>), dim3(mt * nt), dim3(GNT), 0, s,
                        ColMajorAT{a, lda, m}, ColMajorB{b, ldb, n}, m, n, k, alpha, c, ldc, mt, mt * nt);
+    NGW_HIP(hipGetLastError());
+    return NGW_OK;
+}
+
+// C = alpha A^T B (n x n) where the product is symmetric: the 64 x 64 tiles on
+// and above the diagonal, the k sum in S ranges.  2000 columns have 528 such
+// tiles, two or three per CU, and k is the grid: without the ranges the CUs
+// with three set the time (10.5 ms for k = 97,000, now 8.3; the full product on 128 x
+// 128 tiles 11.4).  Range partials lie tile after tile; sym_sum_kernel adds
+// them in order and writes each element and its mirror.
+constexpr int SYM = 64;
+__global__ __launch_bounds__(GNT) void gemm_sym_kernel(ColMajorAT al, ColMajorB bl, int k, int kc, int ntiles,
+                                                       double* part)
+{
+    __shared__ SmemF64<SYM, SYM> sm;
+    const int id = xcd_tile(blockIdx.x, gridDim.x), split = id / ntiles, tile = id - split * ntiles;
+    // tile = tn (tn + 1) / 2 + tm, tm <= tn
+    int tn = (int)((sqrt(8.0 * tile + 1.0) - 1.0) * 0.5);
+    if ((tn + 1) * (tn + 2) / 2 <= tile) ++tn;
+    if (tn * (tn + 1) / 2 > tile) --tn;
+    const long k0 = (long)split * kc;
+    al.a += k0;
+    bl.b += k0;
+    AccF64<SYM, SYM> acc;
+    gemm_f64_tile<SYM, SYM>(al, bl, (tile - tn * (tn + 1) / 2) * SYM, tn * SYM, min(kc, k - (int)k0), acc, sm);
+    double* o = part + (long)id * SYM * SYM;
+    for_acc_f64<SYM, SYM>(acc, [&](int row, int col, double val) { o[row + col * SYM] = val; });
+}
+
+__global__ __launch_bounds__(256) void sym_sum_kernel(const double* part, int S, int ntiles, int n, double alpha,
+                                                      double* c, long ldc)
+{
+    const int tile = blockIdx.x;
+    int tn = (int)((sqrt(8.0 * tile + 1.0) - 1.0) * 0.5);
+    if ((tn + 1) * (tn + 2) / 2 <= tile) ++tn;
+    if (tn * (tn + 1) / 2 > tile) --tn;
+    const int m0 = (tile - tn * (tn + 1) / 2) * SYM, n0 = tn * SYM;
+    for (int e = threadIdx.x; e < SYM * SYM; e += 256) {
+        double s = 0.0;
+        for (int p = 0; p < S; ++p) s += part[((long)p * ntiles + tile) * SYM * SYM + e];
+        const int gm = m0 + e % SYM, gn = n0 + e / SYM;
+        if (gm >= n || gn >= n) continue;
+        const double v = alpha * s;
+        c[gm + (long)gn * ldc] = v;
+        if (m0 != n0) c[gn + (long)gm * ldc] = v;
+    }
+}
+
+int gemm_f64_tn_sym(hipStream_t s, int n, int k, double alpha, const double* a, long lda, const double* b, long ldb,
+                    double* c, long ldc, DevBuf& part)
+{
+    if (n <= 0) return NGW_OK;
+    const int nt = (n + SYM - 1) / SYM, ntiles = nt * (nt + 1) / 2;
+    // about eight workgroups per CU, ranges of at least 2048
+    int S = std::max(1, std::min((2048 + ntiles - 1) / ntiles, k / 2048));
+    const int kc = (k + S - 1) / S;
+    S = (k + kc - 1) / kc;
+    NGW_TRY(part.ensure(sizeof(double) * (size_t)S * ntiles * SYM * SYM));
+    hipLaunchKernelGGL(gemm_sym_kernel, dim3(ntiles * S), dim3(GNT), 0, s, ColMajorAT{a, lda, n}, ColMajorB{b, ldb, n},
+                       k, kc, ntiles, part.as<double>());
+    hipLaunchKernelGGL(sym_sum_kernel, dim3(ntiles), dim3(256), 0, s, part.as<const double>(), S, ntiles, n, alpha, c,
+                       ldc);
     NGW_HIP(hipGetLastError());
     return NGW_OK;
 }
@@ -710,8 +774,6 @@ int operator_f64_one(ngw_context* ctx, const OperatorArgs& a)
 }
 
 // ---------------------------------------------------------------- launchers
-static int tiles(long m, int bm, long n, int bn) { return (int)((m + bm - 1) / bm * ((n + bn - 1) / bn)); }
-
 // Tile choice of the FP64 products.  Every form below adds each element's sum
 // in the same order, so the choice changes no bit of a result.  A lone
 // workgroup per CU needs 0.35 us per 16 k for a 32 x 32 tile, 0.54 us for

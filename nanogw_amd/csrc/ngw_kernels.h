@@ -108,6 +108,8 @@ int gemm_f64(hipStream_t s, int m, int n, int k, const double* a, long lda, cons
              long ldb, double* c, long ldc);
 int gemm_f64_tn(hipStream_t s, int m, int n, int k, double alpha, const double* a, long lda,
                 const double* b, long ldb, double* c, long ldc);
+int gemm_f64_tn_sym(hipStream_t s, int n, int k, double alpha, const double* a, long lda, const double* b, long ldb,
+                    double* c, long ldc, DevBuf& part);
 int k1_slots(int nv);
 int k1_reduce(hipStream_t s, const double* tpart, long ldt, int nmu, int nvec, int nv, double* t);
 int gemm_lowp(hipStream_t s, int kind, int m, int n, int k, const double* a, long lda, const double* b, long ldb,
