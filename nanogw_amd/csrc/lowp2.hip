@@ -48,8 +48,8 @@ __device__ __forceinline__ int find_pre(const int* pre, int nreq, int bid)
 constexpr int L2K2 = 64;
 
 // Tile configurations of the K1 and K3 GEMMs: {BM, BN, D, PM} with D the
-// number of slabs in flight (register prefetch depth) and PM the number of
-// M-groups the 8 XCDs are split into.  XCD x owns the tile rectangle
+// number of slabs in flight (register prefetch depth) and PM the largest number
+// of M-groups the 8 XCDs are split into (xcd_groups).  XCD x owns the tile rectangle
 // (M-group x mod PM) x (N-group x / PM): with PM > 1 each XCD touches only its
 // share of the A operand, which then stays in that XCD's L2, while the tiles
 // of one N column (M fastest inside the rectangle) share their B slab.  Index
@@ -94,10 +94,23 @@ static int cfg_set_prec(int prec) { return prec == PREC_BF16X3 ? 1 : prec == PRE
 constexpr float F16_OPS = 4096.0f, F16_VEC = 16384.0f;
 constexpr double F16_UNSCALE = 1.0 / 67108864.0;
 
+// M-groups of a request: the configuration's, but halved until the M tiles
+// divide among them to within a tenth.  A batched molecule has one to five M
+// tiles: on the configuration's eight (K1) or four (K3) groups half of the
+// XCDs and more had none of them (a batch of three BF16x3 molecules with one to
+// four M tiles: K1 899 -> 476 us, K3 1387 -> 948; one with four in K1 and three
+// in K3, Nv = 37: K1 347 -> 203, K3 469 -> 369; 40 and 12 tiles as before).
+__host__ __device__ inline int xcd_groups(int mt, int pm)
+{
+    while (pm > 1 && 10 * mt < 9 * pm * ((mt + pm - 1) / pm)) pm >>= 1;
+    return pm;
+}
+
 // Workgroups of one request's GEMM: NXCD rectangles of the largest size
 // (workgroups of a smaller rectangle beyond its tiles exit at once).
 __host__ __device__ inline int xcd_grid(int mt, int nt, int pm)
 {
+    pm = xcd_groups(mt, pm);
     const int pn = NXCD / pm;
     return NXCD * ((mt + pm - 1) / pm) * ((nt + pn - 1) / pn);
 }
@@ -107,6 +120,7 @@ __host__ __device__ inline int xcd_grid(int mt, int nt, int pm)
 // false for a workgroup past its rectangle.
 __device__ __forceinline__ bool xcd_rect_tile(int local, int mt, int nt, int pm, int& tm, int& tn)
 {
+    pm = xcd_groups(mt, pm);
     const int pn = NXCD / pm;
     const int x = local % NXCD, i = local / NXCD;
     const int mg = x % pm, ng = x / pm;
