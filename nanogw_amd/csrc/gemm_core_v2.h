@@ -86,9 +86,22 @@ struct alignas(16) SmemV2 {
 // Loads through global-address-space pointers: global_load instructions count
 // only in vmcnt, so the compiler can wait for an older slab while a newer
 // one is still in flight (generic pointers give flat loads, which also count
-// in lgkmcnt and force full waits).
+// in lgkmcnt and force full waits).  The pointers of a request's descriptor come
+// from memory, so the compiler knows nothing of them: every access of the
+// conversion passes and epilogues goes through gptr too (FP64 vectors at Nv = 37:
+// xprep 217 -> 147 us, the BF16x3 K3 369 -> 354; at (5000, 100, 1500) xprep 876 ->
+// 616 and xscale 461 -> 334 us).
 typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
+typedef float f32x2 __attribute__((ext_vector_type(2)));
+typedef double f64x2 __attribute__((ext_vector_type(2)));
 
+template <class T>
+using gptr = T __attribute__((address_space(1)))*;
+template <class T>
+__device__ __forceinline__ gptr<T> as_global(T* p)
+{
+    return (gptr<T>)p;
+}
 template <class T>
 __device__ __forceinline__ T gload(const void* p)
 {

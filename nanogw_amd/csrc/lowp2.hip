@@ -307,14 +307,15 @@ __global__ __launch_bounds__(256) void xscale_kernel(const LpOp* ops, LpOp op1, 
     const long xoff = (long)b * op.ld;
     const long chunk = ((ncv + split - 1) / split + 3) & ~3L;  // a multiple of four elements
     const long lo = part * chunk, hi = min(ncv, lo + chunk);
+    const gptr<const float> xsig = as_global(op.xsig);
     double m = 0.0;
     auto scan = [&](auto* xp) {
         for (long base = lo + threadIdx.x; base < hi; base += 2048) {
             double v[8];
 #pragma unroll
             for (int u = 0; u < 8; ++u) {
-                const long idx = base + 256 * u;
-                v[u] = idx < hi ? fabs((double)xp[xoff + idx]) * (double)op.xsig[idx] : 0.0;
+                const long idx = min(base + 256 * u, hi - 1);  // past the end: the last again
+                v[u] = fabs((double)xp[xoff + idx]) * (double)xsig[idx];
             }
 #pragma unroll
             for (int u = 0; u < 8; ++u) m = fmax(m, v[u]);
@@ -322,21 +323,15 @@ __global__ __launch_bounds__(256) void xscale_kernel(const LpOp* ops, LpOp op1, 
     };
     // FP32 input with 16-byte aligned starts: four elements per load
     auto scan4 = [&](const float* xp) {
-        const float4* x4 = reinterpret_cast<const float4*>(xp + xoff + lo);
-        const float4* s4 = reinterpret_cast<const float4*>(op.xsig + lo);
+        const gptr<const f32x4> x4 = (gptr<const f32x4>)(xp + xoff + lo), s4 = (gptr<const f32x4>)(op.xsig + lo);
         const long nq = hi > lo ? (hi - lo) >> 2 : 0;
         for (long q0 = threadIdx.x; q0 < nq; q0 += 256 * 4) {
-            float4 xv[4], sv[4];
+            f32x4 xv[4], sv[4];
 #pragma unroll
             for (int u = 0; u < 4; ++u) {
-                const long q = q0 + 256 * u;
-                if (q < nq) {
-                    xv[u] = x4[q];
-                    sv[u] = s4[q];
-                } else {
-                    xv[u] = float4{0.0f, 0.0f, 0.0f, 0.0f};
-                    sv[u] = xv[u];
-                }
+                const long q = min(q0 + 256 * u, nq - 1);  // past the end: the last again
+                xv[u] = x4[q];
+                sv[u] = s4[q];
             }
 #pragma unroll
             for (int u = 0; u < 4; ++u) {
@@ -347,7 +342,7 @@ __global__ __launch_bounds__(256) void xscale_kernel(const LpOp* ops, LpOp op1, 
             }
         }
         for (long idx = lo + 4 * nq + threadIdx.x; idx < hi; idx += 256)
-            m = fmax(m, fabs((double)xp[xoff + idx]) * (double)op.xsig[idx]);
+            m = fmax(m, fabs((double)as_global(xp)[xoff + idx]) * (double)xsig[idx]);
     };
     if (x32) {
         const float* xf = reinterpret_cast<const float*>(sg.x);
@@ -355,9 +350,9 @@ __global__ __launch_bounds__(256) void xscale_kernel(const LpOp* ops, LpOp op1, 
             ((reinterpret_cast<uintptr_t>(op.xsig) & 15) == 0))
             scan4(xf);
         else
-            scan(xf);
+            scan(as_global(xf));
     } else {
-        scan(sg.x);
+        scan(as_global(sg.x));
     }
     const float mb = block_max256((float)m);
     if (threadIdx.x == 0) op.xpart[b * XS_SPLIT + part] = mb;
@@ -413,6 +408,7 @@ __global__ __launch_bounds__(256) void xprep_kernel(const LpOp* ops, LpOp op1, c
     // with an exact correction
     const int tot = vn * cn;
     const long base = v0 + (long)c0 * op.nv;
+    const gptr<const float> xsig = as_global(op.xsig);
     const float inv = 1.0f / (float)vn;
     auto walk = [&](auto* xp) {
         for (int e0 = threadIdx.x; e0 < tot; e0 += 256 * 8) {
@@ -420,15 +416,15 @@ __global__ __launch_bounds__(256) void xprep_kernel(const LpOp* ops, LpOp op1, c
             int cc[8], vv[8];
 #pragma unroll
             for (int u = 0; u < 8; ++u) {
-                const int e = e0 + 256 * u;
+                const int e = min(e0 + 256 * u, tot - 1);  // past the end: the last again, not stored
                 int c = (int)((float)e * inv);
                 if (c * vn > e) --c;
                 if ((c + 1) * vn <= e) ++c;
                 cc[u] = c;
                 vv[u] = e - c * vn;
                 const long idx = base + vv[u] + (long)c * op.nv;
-                xv[u] = e < tot ? (double)xp[xoff + idx] : 0.0;
-                sv[u] = e < tot ? (double)op.xsig[idx] : 0.0;
+                xv[u] = (double)xp[xoff + idx];
+                sv[u] = (double)xsig[idx];
             }
 #pragma unroll
             for (int u = 0; u < 8; ++u)
@@ -437,7 +433,7 @@ __global__ __launch_bounds__(256) void xprep_kernel(const LpOp* ops, LpOp op1, c
 #pragma unroll
                 for (int u = 0; u < 8; ++u)
                     if (e0 + 256 * u < tot)
-                        op.q32[(long)b * op.nv * op.nc + base + vv[u] + (long)cc[u] * op.nv] = (float)xv[u];
+                        as_global(op.q32)[(long)b * op.nv * op.nc + base + vv[u] + (long)cc[u] * op.nv] = (float)xv[u];
             }
         }
     };
@@ -445,11 +441,10 @@ __global__ __launch_bounds__(256) void xprep_kernel(const LpOp* ops, LpOp op1, c
     // and of xsig: four elements per 16-byte load when both starts are
     // 16-byte aligned; the last tot mod 4 elements go element-wise.
     auto walk4 = [&](const float* xp) {
-        const float4* x4 = reinterpret_cast<const float4*>(xp + xoff + base);
-        const float4* s4 = reinterpret_cast<const float4*>(op.xsig + base);
+        const gptr<const f32x4> x4 = (gptr<const f32x4>)(xp + xoff + base), s4 = (gptr<const f32x4>)(op.xsig + base);
         const int nq = tot >> 2;
         for (int q0 = threadIdx.x; q0 < nq; q0 += 256 * 4) {
-            float4 xv[4], sv[4];
+            f32x4 xv[4], sv[4];
 #pragma unroll
             for (int u = 0; u < 4; ++u) {
                 const int q = q0 + 256 * u;
@@ -481,7 +476,7 @@ __global__ __launch_bounds__(256) void xprep_kernel(const LpOp* ops, LpOp op1, c
         }
         for (int e = 4 * nq + threadIdx.x; e < tot; e += 256) {
             const int c = e / vn, v = e - c * vn;
-            tile[c * pitch + v] = (float)((double)xp[xoff + base + e] * ((double)op.xsig[base + e] * f16s));
+            tile[c * pitch + v] = (float)((double)as_global(xp)[xoff + base + e] * ((double)xsig[base + e] * f16s));
         }
     };
     if (x32) {
@@ -490,9 +485,9 @@ __global__ __launch_bounds__(256) void xprep_kernel(const LpOp* ops, LpOp op1, c
                              ((reinterpret_cast<uintptr_t>(xf) & 15) == 0) &&
                              ((reinterpret_cast<uintptr_t>(op.xsig) & 15) == 0);
         if (vn == op.nv && aligned) walk4(xf);
-        else walk(xf);
+        else walk(as_global(xf));
     } else {
-        walk(sg.x);
+        walk(as_global(sg.x));
     }
     for (int i = cn * pitch + threadIdx.x; i < ct * pitch; i += 256) tile[i] = 0.0f;  // k padding rows
     __syncthreads();
@@ -507,7 +502,7 @@ __global__ __launch_bounds__(256) void xprep_kernel(const LpOp* ops, LpOp op1, c
         for (int e = 0; e < 8; ++e) w[e] = tile[(cq + e) * pitch + vl];
         const long o = (long)(v0 + vl + op.nv * b) * op.ldc1 + c0 + cq;
         if constexpr (KIND == LP_F32) {
-            f32x4* out = reinterpret_cast<f32x4*>(reinterpret_cast<float*>(op.xlp_hi) + o);
+            const gptr<f32x4> out = (gptr<f32x4>)((float*)op.xlp_hi + o);
             out[0] = f32x4{w[0], w[1], w[2], w[3]};
             out[1] = f32x4{w[4], w[5], w[6], w[7]};
         } else {
@@ -522,9 +517,9 @@ __global__ __launch_bounds__(256) void xprep_kernel(const LpOp* ops, LpOp op1, c
                     lo[e] = (unsigned)la | ((unsigned)lb << 16);
                 }
             }
-            *reinterpret_cast<u32x4*>(reinterpret_cast<E*>(op.xlp_hi) + o) = u32x4{hi[0], hi[1], hi[2], hi[3]};
+            *(gptr<u32x4>)((E*)op.xlp_hi + o) = u32x4{hi[0], hi[1], hi[2], hi[3]};
             if constexpr (V2Traits<KIND>::NSPLIT == 2)
-                *reinterpret_cast<u32x4*>(reinterpret_cast<E*>(op.xlp_lo) + o) = u32x4{lo[0], lo[1], lo[2], lo[3]};
+                *(gptr<u32x4>)((E*)op.xlp_lo + o) = u32x4{lo[0], lo[1], lo[2], lo[3]};
         }
     }
 }
@@ -542,10 +537,10 @@ __global__ __launch_bounds__(256) void red2_kernel(const LpOp* ops, LpOp op1, co
     if (nu < op.nmu && b < op.nvec) {
         const int first = (b * op.nv) / bn, last = ((b + 1) * op.nv - 1) / bn;
         double acc = 0.0;
-        for (int sl = 0; sl <= last - first; ++sl) acc += op.tpart[((long)sl * op.nvec + b) * op.nmu + nu];
+        for (int sl = 0; sl <= last - first; ++sl) acc += as_global(op.tpart)[((long)sl * op.nvec + b) * op.nmu + nu];
         out = (float)acc;
     }
-    op.t32[i] = out;
+    as_global(op.t32)[i] = out;
     if (b == op.nvec) op.u32[i] = 0.0f;
     if (op.umax && nu == 0 && b < op.nvec) op.umax[b] = 0u;  // K2 takes the maximum
 }
@@ -595,11 +590,11 @@ __global__ __launch_bounds__(GNT) void k1v2_kernel(const LpOp* ops, LpOp op1, co
     // (columns past N and rows past ldm1 hold zero sums; their Psi_v loads are
     // clamped, not skipped: a branch around each load would make it wait for
     // the one before)
-    const float* pcol[FN];
+    gptr<const float> pcol[FN];
 #pragma unroll
     for (int j = 0; j < FN; ++j) {
         const int gn = min(n0 + wn + 16 * j + (lane & 15), N - 1);
-        pcol[j] = op.psiv32 + (long)(gn % nv) * op.ldm1;
+        pcol[j] = as_global(op.psiv32) + (long)(gn % nv) * op.ldm1;
     }
 #pragma unroll
     for (int pass = 0; pass < BM / HALF; ++pass) {
@@ -611,7 +606,7 @@ __global__ __launch_bounds__(GNT) void k1v2_kernel(const LpOp* ops, LpOp op1, co
             const int gm0 = min(m0 + row0, op.ldm1 - 4);
             f32x4 pv[FN];
 #pragma unroll
-            for (int j = 0; j < FN; ++j) pv[j] = *reinterpret_cast<const f32x4*>(pcol[j] + gm0);
+            for (int j = 0; j < FN; ++j) pv[j] = *(gptr<const f32x4>)(pcol[j] + gm0);
 #pragma unroll
             for (int j = 0; j < FN; ++j) {
                 const int col = wn + 16 * j + (lane & 15);
@@ -624,7 +619,7 @@ __global__ __launch_bounds__(GNT) void k1v2_kernel(const LpOp* ops, LpOp op1, co
             int row = e % HALF, b = b_lo + e / HALF;
             int c0 = max(n0, b * nv) - n0, c1 = min(nend, (b + 1) * nv) - n0;
             double sc = 1.0;
-            if constexpr (KIND == LP_F16) sc = (double)op.xsc[b] * (double)(1.0f / F16_VEC) * (double)(1.0f / F16_OPS);
+            if constexpr (KIND == LP_F16) sc = (double)as_global(op.xsc)[b] * (double)(1.0f / F16_VEC) * (double)(1.0f / F16_OPS);
             // in column order, eight LDS reads in flight
             float sum = 0.0f;
             int cc = c0;
@@ -640,7 +635,7 @@ __global__ __launch_bounds__(GNT) void k1v2_kernel(const LpOp* ops, LpOp op1, co
             int slot = tn - (b * nv) / BN;
             double t = (double)sum;
             if constexpr (KIND == LP_F16) t *= sc;
-            if (gm < op.nmu) op.tpart[((long)slot * op.nvec + b) * op.nmu + gm] = t;
+            if (gm < op.nmu) as_global(op.tpart)[((long)slot * op.nvec + b) * op.nmu + gm] = t;
         }
     }
 }
@@ -659,7 +654,7 @@ __global__ __launch_bounds__(GNT) void k2v2_kernel(const LpOp* ops, LpOp op1, co
     // loader reads u over the whole padded slab
     for_acc_lp<L2K2, L2K2>(acc, [&](int row, int col, float val) {
         int gm = m0 + row, gn = n0 + col;
-        if (gm < op.ldm1 && gn < op.nvec) op.u32[gm + (long)gn * op.ldm1] = val;
+        if (gm < op.ldm1 && gn < op.nvec) as_global(op.u32)[gm + (long)gn * op.ldm1] = val;
     });
     if constexpr (UMAX) {
         // umax(b) = max_mu |u(mu, b)|: per column over the wave's rows (lanes
@@ -709,7 +704,7 @@ __global__ __launch_bounds__(256) void wprep_kernel(const LpOp* ops, LpOp op1, c
     const float* u = op.u32 + (long)b * op.ldm1 + mu;
     const f32x4 u0 = gload<f32x4>(u), u1 = gload<f32x4>(u + 4);
     float usc = 1.0f;
-    if constexpr (KIND == LP_F16) usc = zero_row ? 1.0f : pow2_ceil(__uint_as_float(op.umax[b]));
+    if constexpr (KIND == LP_F16) usc = zero_row ? 1.0f : pow2_ceil(__uint_as_float(as_global(op.umax)[b]));
     const int vend = zero_row ? 1 : min(WP_V, op.nv - v0);
 #pragma unroll
     for (int dv = 0; dv < WP_V; ++dv) {
@@ -719,15 +714,15 @@ __global__ __launch_bounds__(256) void wprep_kernel(const LpOp* ops, LpOp op1, c
         f32x4 w0 = gload<f32x4>(p) * u0;
         f32x4 w1 = gload<f32x4>(p + 4) * u1;
         if constexpr (KIND == LP_F16) {
-            const float sc = zero_row ? 1.0f : op.vsc[v] * usc;
+            const float sc = zero_row ? 1.0f : as_global(op.vsc)[v] * usc;
             const float f = F16_VEC / sc;
             w0 = w0 * f;
             w1 = w1 * f;
-            if (mu == 0 && !zero_row) op.wsc[j] = sc;
+            if (mu == 0 && !zero_row) as_global(op.wsc)[j] = sc;
         }
         const long o = (long)j * op.ldm1 + mu;
         if constexpr (KIND == LP_F32) {
-            f32x4* out = reinterpret_cast<f32x4*>(reinterpret_cast<float*>(op.wlp_hi) + o);
+            const gptr<f32x4> out = (gptr<f32x4>)((float*)op.wlp_hi + o);
             out[0] = w0;
             out[1] = w1;
         } else {
@@ -743,9 +738,9 @@ __global__ __launch_bounds__(256) void wprep_kernel(const LpOp* ops, LpOp op1, c
                     lo[e] = (unsigned)la | ((unsigned)lb << 16);
                 }
             }
-            *reinterpret_cast<u32x4*>(reinterpret_cast<E*>(op.wlp_hi) + o) = u32x4{hi[0], hi[1], hi[2], hi[3]};
+            *(gptr<u32x4>)((E*)op.wlp_hi + o) = u32x4{hi[0], hi[1], hi[2], hi[3]};
             if constexpr (V2Traits<KIND>::NSPLIT == 2)
-                *reinterpret_cast<u32x4*>(reinterpret_cast<E*>(op.wlp_lo) + o) = u32x4{lo[0], lo[1], lo[2], lo[3]};
+                *(gptr<u32x4>)((E*)op.wlp_lo + o) = u32x4{lo[0], lo[1], lo[2], lo[3]};
         }
     }
 }
@@ -753,14 +748,14 @@ __global__ __launch_bounds__(256) void wprep_kernel(const LpOp* ops, LpOp op1, c
 // 16-byte accesses of four consecutive elements (FP32 or FP64), widened to
 // or narrowed from FP64.
 __device__ __forceinline__ bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
-__device__ __forceinline__ void st4(float* p, const double (&r)[4])
+__device__ __forceinline__ void st4(gptr<float> p, const double (&r)[4])
 {
-    *reinterpret_cast<f32x4*>(p) = f32x4{(float)r[0], (float)r[1], (float)r[2], (float)r[3]};
+    *(gptr<f32x4>)p = f32x4{(float)r[0], (float)r[1], (float)r[2], (float)r[3]};
 }
-__device__ __forceinline__ void st4(double* p, const double (&r)[4])
+__device__ __forceinline__ void st4(gptr<double> p, const double (&r)[4])
 {
-    reinterpret_cast<double2*>(p)[0] = double2{r[0], r[1]};
-    reinterpret_cast<double2*>(p)[1] = double2{r[2], r[3]};
+    ((gptr<f64x2>)p)[0] = f64x2{r[0], r[1]};
+    ((gptr<f64x2>)p)[1] = f64x2{r[2], r[3]};
 }
 
 // 128 x 128 tiles keep three workgroups per CU: the register budget is 168
@@ -793,31 +788,31 @@ void k3v2_kernel(const LpOp* ops, LpOp op1, const LpStage* st, LpStage st1,
     // epilogue: OperatorEpilogue's stage (diagonal term, Horner / Clenshaw
     // combination, Lanczos accumulate), written out for one leading
     // dimension shared by every vector block of the request
-    const float2* dp = op.dpair;
+    const gptr<const f32x2> dp = (gptr<const f32x2>)op.dpair;
     const double beta = op.tda ? 2.0 : 4.0;
     const bool acc_on = sg.accumulate == 1 || (sg.accumulate == 2 && *op.kstep > 1);
     const bool use_q = op.q != nullptr && sg.gamma != 0.0;
     const long ncv = (long)nv * op.nc;
-    const float* sigc = op.sig + nv;
+    const gptr<const float> sigc = as_global(op.sig) + nv;
     // element types of x, y, out fixed at compile time per flag combination
     auto epi = [&](auto xt, auto yt, auto ot) {
         typedef decltype(xt) TX;
         typedef decltype(yt) TY;
         typedef decltype(ot) TO;
-        const TX* xp = reinterpret_cast<const TX*>(sg.x);
-        const TY* yp = reinterpret_cast<const TY*>(sg.y);
-        TO* op_ = reinterpret_cast<TO*>(sg.out);
+        const gptr<const TX> xp = (gptr<const TX>)sg.x;
+        const gptr<const TY> yp = (gptr<const TY>)sg.y;
+        const gptr<TO> op_ = (gptr<TO>)sg.out;
         // FP32 output stages (ST_O32 comes with ST_Q32) read the first
         // stage's FP32 copy of q
         typedef std::conditional_t<sizeof(TO) == 4, float, double> TQ;
-        const TQ* qp;
-        if constexpr (sizeof(TO) == 4) qp = op.q32;
-        else qp = op.q;
+        gptr<const TQ> qp;
+        if constexpr (sizeof(TO) == 4) qp = as_global(op.q32);
+        else qp = as_global(op.q);
         // four consecutive pairs icv = v..v+3 of one c share a b when nv is a
         // multiple of four (tiles start at multiples of four): then every
         // array is read and written with 16-byte accesses
-        const bool vec = (nv & 3) == 0 && (op.ld & 3) == 0 && aligned16(xp) && aligned16(yp) && aligned16(op_) &&
-                         aligned16(use_q ? qp : nullptr) && aligned16(dp) &&
+        const bool vec = (nv & 3) == 0 && (op.ld & 3) == 0 && aligned16(sg.x) && aligned16(sg.y) && aligned16(sg.out) &&
+                         (!use_q || aligned16(sizeof(TO) == 4 ? (const void*)op.q32 : op.q)) && aligned16(op.dpair) &&
                          (KIND != LP_F16 || aligned16(op.wsc)) && (ncv & 3) == 0;
         // The tile passes through LDS one accumulator fragment row at a time:
         // in pass q every wave writes its fragment row q (16 tile rows, so
@@ -859,12 +854,12 @@ void k3v2_kernel(const LpOp* ops, LpOp op1, const LpStage* st, LpStage st1,
                 if ((int)threadIdx.x >= RS * BN || j >= N) return;
                 const int b = j / nv, v = j - b * nv, rl0 = (int)threadIdx.x / BN;
                 const long boff = (long)b * op.ld;
-                const TX* xb = xp + boff;
-                const TY* yb = yp + boff;
-                const TQ* qb = qp + (sizeof(TQ) == 4 ? (long)b * ncv : boff);
-                TO* ob = op_ + boff;
+                const gptr<const TX> xb = xp + boff;
+                const gptr<const TY> yb = yp + boff;
+                const gptr<const TQ> qb = qp + (sizeof(TQ) == 4 ? (long)b * ncv : boff);
+                const gptr<TO> ob = op_ + boff;
                 double wsj = 1.0;
-                if constexpr (KIND == LP_F16) wsj = (double)op.wsc[j] * F16_UNSCALE;
+                if constexpr (KIND == LP_F16) wsj = (double)as_global(op.wsc)[j] * F16_UNSCALE;
 #pragma unroll 1
                 for (int k0 = 0; k0 < EPR / RS; k0 += EB) {
                     TX xv[EB];
@@ -872,7 +867,7 @@ void k3v2_kernel(const LpOp* ops, LpOp op1, const LpStage* st, LpStage st1,
                     TQ qv[EB];
                     TO av[EB];
                     float sc[EB];
-                    float2 f[EB];
+                    f32x2 f[EB];
                     // rows past the operand read its last row
                     auto row = [&](int k) {
                         const int rl = rl0 + RS * (k0 + k);
@@ -935,13 +930,13 @@ void k3v2_kernel(const LpOp* ops, LpOp op1, const LpStage* st, LpStage st1,
                     const int b = jc / nv, idx = jc - b * nv + cc * nv;
                     ii[g] = idx + (long)b * op.ld;
                     sc[g] = sigc[cc];
-                    if constexpr (KIND == LP_F16) ws[g] = *reinterpret_cast<const f32x4*>(op.wsc + jc);
-                    xr[g] = *reinterpret_cast<const x4*>(xp + ii[g]);
-                    d01[g] = *reinterpret_cast<const f32x4*>(dp + idx);
-                    d23[g] = *reinterpret_cast<const f32x4*>(dp + idx + 2);
-                    if (yp) yr[g] = *reinterpret_cast<const y4*>(yp + ii[g]);
-                    if (use_q) qr[g] = *reinterpret_cast<const q4*>(qp + (sizeof(TQ) == 4 ? idx + (long)b * ncv : ii[g]));
-                    if (acc_on) ar[g] = *reinterpret_cast<const o4*>(op_ + ii[g]);
+                    if constexpr (KIND == LP_F16) ws[g] = gload<f32x4>(op.wsc + jc);
+                    xr[g] = *(gptr<const x4>)(xp + ii[g]);
+                    d01[g] = *(gptr<const f32x4>)(dp + idx);
+                    d23[g] = *(gptr<const f32x4>)(dp + idx + 2);
+                    if (yp) yr[g] = *(gptr<const y4>)(yp + ii[g]);
+                    if (use_q) qr[g] = *(gptr<const q4>)(qp + (sizeof(TQ) == 4 ? idx + (long)b * ncv : ii[g]));
+                    if (acc_on) ar[g] = *(gptr<const o4>)(op_ + ii[g]);
                 }
 #pragma unroll
                 for (int g = 0; g < GU; ++g) {
