@@ -380,6 +380,7 @@ int rebuild_group(ngw_batch* b)
     std::vector<GOp> ops(nreq);
     std::vector<GStage> stages((size_t)nreq * npoly);
     std::vector<LpOp> lops(nreq);
+    LpTileRule rule;
     std::vector<LpStage> lstages((size_t)nreq * npoly);
     std::vector<GLz> lz(nreq);
     std::vector<int> pre((NTAB_AB + 1) * (nreq + 1), 0);
@@ -436,11 +437,17 @@ int rebuild_group(ngw_batch* b)
                 lstages[(size_t)i * npoly + sgi] = LpStage{p.x, p.out, p.y, p.alpha, p.bx, p.by, p.gamma,
                                                            p.accumulate ? 2 : 0, p.flags};
             }
-            int tot[LP_NKERNEL];
-            lp2_grid_counts(prec, b->lp_c1, b->lp_c3, d, tot);
-            for (int k = 0; k < LP_NKERNEL; ++k) P(k, i + 1) = P(k, i) + tot[k];
+            rule.add(d);
         }
         P(NTAB_AB, i + 1) = P(NTAB_AB, i) + B;
+    }
+    if (prec != PREC_F64) {
+        rule.pick(prec, b->lp_c1, b->lp_c3);
+        for (int i = 0; i < nreq; ++i) {
+            int tot[LP_NKERNEL];
+            lp2_grid_counts(prec, b->lp_c1, b->lp_c3, lops[i], tot);
+            for (int k = 0; k < LP_NKERNEL; ++k) P(k, i + 1) = P(k, i) + tot[k];
+        }
     }
     hipStream_t s = b->ctx->stream;
     if (prec == PREC_F64) {

@@ -53,8 +53,9 @@ constexpr int L2K2 = 64;
 // (M-group x mod PM) x (N-group x / PM): with PM > 1 each XCD touches only its
 // share of the A operand, which then stays in that XCD's L2, while the tiles
 // of one N column (M fastest inside the rectangle) share their B slab.  Index
-// 0 is the default; the autotuner (ngw_autotune) times all of them on the
-// caller's shape.
+// 0 is the default (for large FP16 launches it stands for a wider tile with the
+// same results, see LpTileRule::pick); the autotuner (ngw_autotune) times all of
+// them on the caller's shape.
 struct LpCfg {
     int bm, bn, d, pm;
     int fw = 0;  // K3 only: 1 = W formed in the slab loader (no wprep pass)
@@ -74,9 +75,9 @@ constexpr LpCfg K1_CFG[3][LP_NCFG] = {
 // M-group.  FP16 K1 index 4 and K3 indices 4 and 5 are 128 x 256 tiles: per
 // slab a workgroup moves 24 KB into LDS and its four 64 x 128 wave tiles read
 // 48 KB for 128 MFMAs, 576 LDS bytes per MFMA against 768 for 128 x 128 and
-// 640 for 128 x 192.  Which tile wins depends on the shape; K3's result does
-// not (each element sums its K range in the same order in every tile), K1's
-// does through its per-BN partial-sum slots.
+// 640 for 128 x 192.  Which tile wins depends on the shape; the results do not
+// (each element sums its K range in the same order in every tile, and K1's
+// partial sums are those of 128 columns in every tile of 128 and more).
 constexpr LpCfg K3_CFG[3][LP_NCFG] = {
     {{128, 128, 2, 4}, {128, 128, 2, 4, 0, 1}, {128, 128, 2, 4, 1}, {128, 128, 2, 8, 1, 1},
      {128, 128, 2, 2, 0, 1}, {128, 128, 2, 1, 0, 1}},
@@ -560,14 +561,52 @@ __device__ __forceinline__ void lp_gemm(const OperandV2<KIND>& A, const OperandV
     else gemm_v2_tile<KIND, BM, BN, D>(A, B, m0, n0, Kpad, acc, sm);
 }
 
+// Columns of a K1 partial sum: a 256-column tile writes two slots, so the sums
+// (FP32 within a slot, FP64 over slots) are those of the 128-column tiles.
+__host__ __device__ constexpr int k1_slot_cols(int bn) { return bn < 128 ? bn : 128; }
+
+// p[c0] + ... + p[c1 - 1] from left to right, p 16-byte aligned.  One chain of
+// additions, so the LDS reads run ahead of it: sixteen columns are read while
+// the sixteen before are added.
+__device__ __forceinline__ float row_sum(const float* p, int c0, int c1)
+{
+    float sum = 0.0f;
+    int c = c0;
+    for (; (c & 3) && c < c1; ++c) sum += p[c];
+    const int blocks = (c1 - c) / 16;
+    if (c1 - c >= 16) {
+        f32x4 w[4], x[4];
+#pragma unroll
+        for (int k = 0; k < 4; ++k) w[k] = *reinterpret_cast<const f32x4*>(p + c + 4 * k);
+        for (int t = 0; t < blocks; ++t) {
+            const int cn = t + 1 < blocks ? c + 16 : c;
+#pragma unroll
+            for (int k = 0; k < 4; ++k) x[k] = *reinterpret_cast<const f32x4*>(p + cn + 4 * k);
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                sum += w[k].x;
+                sum += w[k].y;
+                sum += w[k].z;
+                sum += w[k].w;
+            }
+#pragma unroll
+            for (int k = 0; k < 4; ++k) w[k] = x[k];
+            c += 16;
+        }
+    }
+    for (; c < c1; ++c) sum += p[c];
+    return sum;
+}
+
 template <int KIND, int BM, int BN, int D, int PM, int SW>
 __global__ __launch_bounds__(GNT) void k1v2_kernel(const LpOp* ops, LpOp op1, const int* pre, int nreq)
 {
     typedef typename V2Traits<KIND>::elem E;
     constexpr int HALF = BM < 64 ? BM : 64;  // rows reduced per LDS pass (keeps the buffer within the slabs' LDS)
+    constexpr int SB = k1_slot_cols(BN);
     __shared__ union {
         LpSmem<KIND, BM, BN, D, SW> ab;
-        float red[HALF][BN + 1];
+        float red[HALF][BN + 4];  // rows 16-byte aligned, 64 lanes' reads of a column or of four on all banks
     } sm;
     LP_PICK_OP();
     const int nv = op.nv, N = nv * op.nvec;
@@ -578,9 +617,6 @@ __global__ __launch_bounds__(GNT) void k1v2_kernel(const LpOp* ops, LpOp op1, co
     lp_gemm<KIND, BM, BN, D, SW>(OperandV2<KIND>{(const E*)op.pct_hi, (const E*)op.pct_lo, op.ldc1, op.nmu},
                                  OperandV2<KIND>{(const E*)op.xlp_hi, (const E*)op.xlp_lo, op.ldc1, N}, m0, n0,
                                  op.ldc1, acc, sm.ab);
-    const int nend = min(n0 + BN, N);
-    const int b_lo = n0 / nv, b_hi = (nend - 1) / nv;
-    const int nbt = b_hi - b_lo + 1;
     // T(mu, j) Psi_v(mu, v(j)): a lane's accumulator fragment holds four
     // consecutive mu of one column j, so Psi_v comes as one 16-byte load from
     // the [v][mu] copy (zero for nmu <= mu < ldm1); v(j) once per column
@@ -615,27 +651,23 @@ __global__ __launch_bounds__(GNT) void k1v2_kernel(const LpOp* ops, LpOp op1, co
             }
         }
         __syncthreads();
-        for (int e = threadIdx.x; e < HALF * nbt; e += GNT) {
-            int row = e % HALF, b = b_lo + e / HALF;
-            int c0 = max(n0, b * nv) - n0, c1 = min(nend, (b + 1) * nv) - n0;
-            double sc = 1.0;
-            if constexpr (KIND == LP_F16) sc = (double)as_global(op.xsc)[b] * (double)(1.0f / F16_VEC) * (double)(1.0f / F16_OPS);
-            // in column order, eight LDS reads in flight
-            float sum = 0.0f;
-            int cc = c0;
-            for (; cc + 8 <= c1; cc += 8) {
-                float w[8];
-#pragma unroll
-                for (int k = 0; k < 8; ++k) w[k] = sm.red[row][cc + k];
-#pragma unroll
-                for (int k = 0; k < 8; ++k) sum += w[k];
+        // sums over each vector's columns within each slot of SB columns, one
+        // (row, vector, slot) per thread, in column order
+        for (int h = 0, e = threadIdx.x; h < BN / SB; ++h) {
+            const int s0 = n0 + SB * h, s1 = min(s0 + SB, N);
+            if (s0 >= N) break;
+            const int b_lo = s0 / nv, items = HALF * ((s1 - 1) / nv - b_lo + 1);
+            for (; e < items; e += GNT) {
+                const int row = e % HALF, b = b_lo + e / HALF;
+                const int c0 = max(s0, b * nv) - n0, c1 = min(s1, (b + 1) * nv) - n0;
+                const int gm = m0 + pass * HALF + row;
+                double sc = 1.0;
+                if constexpr (KIND == LP_F16) sc = (double)as_global(op.xsc)[b] * (double)(1.0f / F16_VEC) * (double)(1.0f / F16_OPS);
+                double t = (double)row_sum(sm.red[row], c0, c1);
+                if constexpr (KIND == LP_F16) t *= sc;
+                if (gm < op.nmu) as_global(op.tpart)[((long)(s0 / SB - (b * nv) / SB) * op.nvec + b) * op.nmu + gm] = t;
             }
-            for (; cc < c1; ++cc) sum += sm.red[row][cc];
-            int gm = m0 + pass * HALF + row;
-            int slot = tn - (b * nv) / BN;
-            double t = (double)sum;
-            if constexpr (KIND == LP_F16) t *= sc;
-            if (gm < op.nmu) as_global(op.tpart)[((long)slot * op.nvec + b) * op.nmu + gm] = t;
+            e -= items;  // the next slot's items go on with the threads that are free
         }
     }
 }
@@ -1038,7 +1070,7 @@ static int lp_launch(hipStream_t st, int c1, int c3, const LpOp* ops, const LpOp
     {
         ProfScope ps(prof, KC_CONVERT);
         hipLaunchKernelGGL(red2_kernel, dim3(tot[3]), dim3(256), 0, st, ops, op1, pre[3], nreq,
-                           K1_CFG[cfg_set(KIND)][c1].bn);
+                           k1_slot_cols(K1_CFG[cfg_set(KIND)][c1].bn));
     }
     {
         ProfScope ps(prof, KC_K2);
@@ -1143,6 +1175,30 @@ void lp2_fill(const ngw_context* op, int kind, int nvec, long ld, int tda, char*
     d.q = nullptr; d.w = nullptr; d.a = nullptr; d.b = nullptr; d.niter = 0; d.kstep = nullptr;
 }
 
+// Tiles of a launch whose configuration index is 0: 128 x 256 for FP16 launches
+// of two such tiles per CU and more, if k is deep enough for the longer
+// epilogue and the LDS of the third buffer to pay: fewer bytes through LDS and
+// L2 per MFMA.  Measured us, 128 x 128 and 128 x 256, K1 / K3 at Nmu, Nv, Nc and
+// vectors: (5000, 100, 1500) 1200: 2265 -> 2008 / 2847 -> 2425, 128: 254 -> 232 /
+// 336 -> 332, 48 (760 / 228 tiles): 101 -> 92 / 137 (181); (2000, 40, 400) 1200:
+// 153 (157), K1's k = 448 / 232 -> 209; (444, 37, 370) 1200: 44 (45) / 103 (124).
+constexpr int BIG_TILES = 512, BIG_K = 1024;
+static_assert(K1_CFG[2][4].bn == 256 && K3_CFG[2][5].bn == 256, "FP16 configurations for large launches");
+void LpTileRule::add(const LpOp& d)
+{
+    const long nt = ((long)d.nv * d.nvec + 255) / 256;
+    tiles1 += (d.nmu + 127) / 128 * nt;
+    tiles3 += (d.nc + 127) / 128 * nt;
+    k1 = std::min(k1, d.ldc1);
+    k3 = std::min(k3, d.ldm1);
+}
+void LpTileRule::pick(int kind, int& c1, int& c3) const
+{
+    if (kind != PREC_F16) return;
+    if (c1 == 0 && tiles1 >= BIG_TILES && k1 >= BIG_K) c1 = 4;
+    if (c3 == 0 && tiles3 >= BIG_TILES && k3 >= BIG_K) c3 = 5;
+}
+
 void lp2_grid_counts(int kind, int c1, int c3, const LpOp& d, int* tot)
 {
     LpGrid g = lp_grid(kind, c1, c3, d.nmu, d.nv, d.nc, d.nvec, d.ldc1, d.ldm1);
@@ -1166,7 +1222,10 @@ int operator_lp2(ngw_context* ctx, const OperatorArgs& a)
         return fail(NGW_ERR_ARG, "low-precision operator needs one leading dimension and acc == out");
     d.q = const_cast<double*>(a.v0);
     LpStage st{a.x, a.out, a.y, a.alpha, a.bx, a.by, a.v0 ? a.gamma : 0.0, a.acc ? 1 : 0, a.flags};
-    const int c1 = ctx->lp_cfg[kind][0], c3 = ctx->lp_cfg[kind][1];
+    int c1 = ctx->lp_cfg[kind][0], c3 = ctx->lp_cfg[kind][1];
+    LpTileRule rule;
+    rule.add(d);
+    rule.pick(kind, c1, c3);
     int tot[LP_NKERNEL];
     lp2_grid_counts(kind, c1, c3, d, tot);
     const int* pre[LP_NKERNEL] = {};

@@ -37,3 +37,27 @@ def test_every_tile_is_computed_once(ngw_ctx, prec, nmu, nc, nv, blksz):
     d = ((e[nv:, None] - e[None, :nv]).reshape(-1))[:, None] * x
     ref = _operator(psi, m, e, nv, x, True) - d
     assert np.abs(y - d - ref).max() < TOL[prec] * np.abs(ref).max()
+
+
+@pytest.mark.parametrize("nmu,nc,nv,blksz", [
+    (1100, 1030, 33, 500),   # wide K1 and K3 tiles, remainders in M and N
+    (1100, 700, 20, 1000),   # k of K1 too short, K3 wide
+    (900, 1281, 129, 117),   # K1 wide (an odd nv above one slot), k of K3 too short
+])
+def test_wide_tiles_do_not_change_a_column(ngw_ctx, nmu, nc, nv, blksz):
+    """Large FP16 calls take 256-column tiles: the bits of a column are those
+    of a narrow call, which takes the 128-column ones."""
+    psi, m, e = _system(nmu, nv, nc, nmu + nc)
+    m *= nmu
+    x = np.random.default_rng(blksz).normal(size=(nv * nc, blksz))
+    ngw_ctx.set_isdf(psi, m, e, nv)
+    ngw_ctx.set_precision("f16")
+    try:
+        wide = ngw_ctx.matvec_isdf_BLOCK(x)
+        narrow = ngw_ctx.matvec_isdf_BLOCK(x[:, :9])
+    finally:
+        ngw_ctx.set_precision("f64")
+    assert np.array_equal(wide[:, :9], narrow)
+    d = ((e[nv:, None] - e[None, :nv]).reshape(-1) ** 2)[:, None] * x[:, -12:]
+    ref = _operator(psi, m, e, nv, x[:, -12:], False) - d
+    assert np.abs(wide[:, -12:] - d - ref).max() < TOL["f16"] * np.abs(ref).max()
