@@ -534,10 +534,13 @@ struct PoissonParity {
         p.vw = vw.as<double>();
         hipLaunchKernelGGL(pt_weights_kernel, dim3(1024), dim3(256), 0, s, p, hp, h, trunc, vw.as<double>());
         NGW_HIP(hipGetLastError());
+        // (the attribute belongs to the kernel, not to this call: always the
+        // largest plane, so that no thread lowers another's limit)
+        constexpr int LDS_MAX = 160 * 1024;
         NGW_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(k->fwd), hipFuncAttributeMaxDynamicSharedMemorySize,
-                                    (int)lds));
+                                    LDS_MAX));
         NGW_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(k->inv), hipFuncAttributeMaxDynamicSharedMemorySize,
-                                    (int)lds));
+                                    LDS_MAX));
         return NGW_OK;
     }
     int run(hipStream_t s, const double* z, long ldz, int ngrid, int cb, double* vz)
