@@ -11,7 +11,7 @@
 //   A^-1      by Cholesky (rocSOLVER potrf + potri; LU getrf + getri when A
 //             is not numerically positive definite)
 //   per block of grid rows R:
-//     B(R, :) = (Psi_v(R, :) G_v) o (Psi(R, :) G)
+//     B(R, :) = (Psi_v(R, :) G_v) o (Psi(R, :) G)   one kernel, both factors in registers
 //     zeta(R, :) = B(R, :) A^-1
 // The products are the library's FP64 MFMA GEMM; the factorization is a
 // plain library call on an n_intp x n_intp matrix (n_intp^3 / 3 FLOP).
@@ -65,13 +65,6 @@ __global__ void symmetrize_lower_kernel(double* a, int n)
     }
 }
 
-// x(r, c) *= y(r, c), both (rows x cols) with leading dimension rows
-__global__ void hadamard_inplace_kernel(double* x, const double* y, long total)
-{
-    for (long t = blockIdx.x * (long)blockDim.x + threadIdx.x; t < total; t += (long)gridDim.x * blockDim.x)
-        x[t] *= y[t];
-}
-
 int rb_check(rocblas_status st, const char* what)
 {
     if (st != rocblas_status_success) return fail(NGW_ERR_HIP, std::string(what) + " failed (rocblas status " +
@@ -87,7 +80,7 @@ int isdf_zeta_dev(ngw_context* ctx, int ngrid, int nband, int nval, const double
 {
     hipStream_t s = ctx->stream;
     const int n = n_intp;
-    DevBuf dint, g, p, q, a, diag, info, b1, b2, ipiv;
+    DevBuf dint, g, p, q, a, diag, info, b1, ipiv;
     NGW_TRY(dint.ensure(sizeof(int) * (size_t)n));
     NGW_TRY(g.ensure(sizeof(double) * (size_t)nband * n));
     NGW_TRY(p.ensure(sizeof(double) * (size_t)n * n));
@@ -153,14 +146,10 @@ int isdf_zeta_dev(ngw_context* ctx, int ngrid, int nband, int nval, const double
     // zeta, block of R grid rows at a time
     const int R = (int)std::min<long>(ngrid, 32768);
     NGW_TRY(b1.ensure(sizeof(double) * (size_t)R * n));
-    NGW_TRY(b2.ensure(sizeof(double) * (size_t)R * n));
     for (int r0 = 0; r0 < ngrid; r0 += R) {
         const int rows = std::min(R, ngrid - r0);
-        NGW_TRY(gemm_f64(s, rows, n, nval, d_psi + r0, ld_psi, g.as<double>(), nband, b1.as<double>(), rows));
-        NGW_TRY(gemm_f64(s, rows, n, nband, d_psi + r0, ld_psi, g.as<double>(), nband, b2.as<double>(), rows));
-        hipLaunchKernelGGL(hadamard_inplace_kernel, dim3(1024), dim3(256), 0, s, b1.as<double>(), b2.as<double>(),
-                           (long)rows * n);
-        NGW_HIP(hipGetLastError());
+        NGW_TRY(gemm_f64_pair(s, rows, n, nval, nband, d_psi + r0, ld_psi, g.as<double>(), nband, b1.as<double>(),
+                              rows));
         NGW_TRY(gemm_f64(s, rows, n, n, b1.as<double>(), rows, a.as<double>(), n, d_zeta + r0, ld_zeta));
     }
     NGW_HIP(hipStreamSynchronize(s));  // workspaces are freed on return

@@ -106,6 +106,9 @@ struct OperatorArgs {
 
 int gemm_f64(hipStream_t s, int m, int n, int k, const double* a, long lda, const double* b,
              long ldb, double* c, long ldc);
+// c = (a(:, :k1) b(:k1, :)) o (a b), element by element, k1 <= k
+int gemm_f64_pair(hipStream_t s, int m, int n, int k1, int k, const double* a, long lda, const double* b, long ldb,
+                  double* c, long ldc);
 int gemm_f64_tn(hipStream_t s, int m, int n, int k, double alpha, const double* a, long lda,
                 const double* b, long ldb, double* c, long ldc);
 int gemm_f64_tn_sym(hipStream_t s, int n, int k, double alpha, const double* a, long lda, const double* b, long ldb,

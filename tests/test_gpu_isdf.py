@@ -105,3 +105,23 @@ def test_cvt_points_vs_oracle(ngw_ctx):
         assert len(set(got.tolist())) == n_intp and got.min() >= 0 and got.max() < len(gidx)
         assert it == it_ref
         assert np.array_equal(got, ref)
+
+
+@pytest.mark.parametrize("n, nv, nband", [(1, 1, 1), (15, 3, 7), (63, 12, 60), (64, 16, 48), (65, 60, 60), (130, 12, 61), (257, 17, 80)])
+def test_zeta_tile_edges(ngw_ctx, n, nv, nband):
+    """B's kernel (both products of a tile in registers) at the edges of its
+    tiles and of its k slabs, nv = nband among them.  Forward error of a solve
+    by an inverse, relative to the largest entry: n eps cond(A) times a small
+    constant."""
+    rng = np.random.default_rng(n)
+    ngrid = 333
+    psi = rng.normal(size=(ngrid, nband))
+    intp = np.sort(rng.choice(ngrid, n, replace=False)).astype(np.int64)
+    zeta, used_lu = ngw_ctx.isdf_zeta(psi, intp, nv)
+    a = (psi[intp, :nv] @ psi[intp, :nv].T) * (psi[intp] @ psi[intp].T)
+    b = (psi[:, :nv] @ psi[intp, :nv].T) * (psi @ psi[intp].T)
+    ref = np.linalg.solve(a, b.T).T
+    tol = 16 * n * np.finfo(float).eps * np.linalg.cond(a)
+    print(n, "zeta vs numpy:", rel_err(zeta, ref), "tol", tol)
+    assert not used_lu
+    assert rel_err(zeta, ref) < tol
