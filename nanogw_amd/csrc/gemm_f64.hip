@@ -24,30 +24,44 @@ namespace ngw {
 static int tiles(long m, int bm, long n, int bn) { return (int)((m + bm - 1) / bm * ((n + bn - 1) / bn)); }
 
 // ---------------------------------------------------------------- plain GEMMs
-template <class AL, class BL>
+template <int BM, int BN, class AL, class BL>
 __global__ __launch_bounds__(GNT) void gemm_plain_kernel(AL al, BL bl, int m, int n, int k, double alpha,
                                                          double* c, long ldc, int mtiles, int ntiles)
 {
-    __shared__ SmemF64<128, 128> sm;
+    __shared__ SmemF64<BM, BN> sm;
     const int tile = xcd_tile(blockIdx.x, ntiles);
-    const int m0 = (tile % mtiles) * 128, n0 = (tile / mtiles) * 128;
-    AccF64<128, 128> acc;
-    gemm_f64_tile<128, 128>(al, bl, m0, n0, k, acc, sm);
-    for_acc_f64<128, 128>(acc, [&](int row, int col, double val) {
+    const int m0 = (tile % mtiles) * BM, n0 = (tile / mtiles) * BN;
+    AccF64<BM, BN> acc;
+    gemm_f64_tile<BM, BN>(al, bl, m0, n0, k, acc, sm);
+    for_acc_f64<BM, BN>(acc, [&](int row, int col, double val) {
         int gm = m0 + row, gn = n0 + col;
         if (gm < m && gn < n) c[gm + (long)gn * ldc] = alpha * val;
     });
 }
 
+// Tiles of 64 x 128 (two waves per SIMD; TF/s, in brackets 128 x 128 with one:
+// 67.2 (64.1) at 31461 x 2000 x 2000, 70.9 (69.1) at 4096^3, 55.8 (54.2) at
+// 32768 x 480 x 480; 128 x 64 64.0, 66.9, 53.4), of 64 x 64 where the wide ones
+// are fewer than the CUs (500 x 480 x 480: 30 us, 44 on 64 x 128, 74 on 128 x
+// 128).  All tiles add a sum in the same order: the same bits.
+template <class AL, class BL>
+static int gemm_plain(hipStream_t s, const AL& al, const BL& bl, int m, int n, int k, double alpha, double* c, long ldc)
+{
+    auto go = [&](auto kernel, int bn) {
+        const int mt = (m + 63) / 64, nt = (n + bn - 1) / bn;
+        hipLaunchKernelGGL(kernel, dim3(mt * nt), dim3(GNT), 0, s, al, bl, m, n, k, alpha, c, ldc, mt, mt * nt);
+    };
+    if (m <= 0 || n <= 0) return NGW_OK;
+    if (tiles(m, 64, n, 128) < 256) go(gemm_plain_kernel<64, 64, AL, BL>, 64);
+    else go(gemm_plain_kernel<64, 128, AL, BL>, 128);
+    NGW_HIP(hipGetLastError());
+    return NGW_OK;
+}
+
 int gemm_f64(hipStream_t s, int m, int n, int k, const double* a, long lda, const double* b,
              long ldb, double* c, long ldc)
 {
-    if (m <= 0 || n <= 0) return NGW_OK;
-    int mt = (m + 127) / 128, nt = (n + 127) / 128;
-    hipLaunchKernelGGL((gemm_plain_kernel<ColMajorA, ColMajorB>), dim3(mt * nt), dim3(GNT), 0, s,
-                       ColMajorA{a, lda, m}, ColMajorB{b, ldb, n}, m, n, k, 1.0, c, ldc, mt, mt * nt);
-    NGW_HIP(hipGetLastError());
-    return NGW_OK;
+    return gemm_plain(s, ColMajorA{a, lda, m}, ColMajorB{b, ldb, n}, m, n, k, 1.0, c, ldc);
 }
 
 // C = (A(:, :k1) B(:k1, :)) o (A B): the two products of a tile one after the
@@ -90,12 +104,7 @@ int gemm_f64_pair(hipStream_t s, int m, int n, int k1, int k, const double* a, l
 int gemm_f64_tn(hipStream_t s, int m, int n, int k, double alpha, const double* a, long lda,
                 const double* b, long ldb, double* c, long ldc)
 {
-    if (m <= 0 || n <= 0) return NGW_OK;
-    int mt = (m + 127) / 128, nt = (n + 127) / 128;
-    hipLaunchKernelGGL((gemm_plain_kernel<ColMajorAT, ColMajorB>), dim3(mt * nt), dim3(GNT), 0, s,
-                       ColMajorAT{a, lda, m}, ColMajorB{b, ldb, n}, m, n, k, alpha, c, ldc, mt, mt * nt);
-    NGW_HIP(hipGetLastError());
-    return NGW_OK;
+    return gemm_plain(s, ColMajorAT{a, lda, m}, ColMajorB{b, ldb, n}, m, n, k, alpha, c, ldc);
 }
 
 // C = alpha A^T B (n x n) where the product is symmetric: the 64 x 64 tiles on

@@ -82,3 +82,21 @@ def test_block_size_does_not_change_a_column(ngw_ctx):
     x = np.random.default_rng(700).normal(size=(nv * nc, 700))
     for n in (2, 30, 333):
         assert np.array_equal(ngw_ctx.matvec_isdf_BLOCK(x[:, :n]), wide[:, :n]), n
+
+
+@pytest.mark.parametrize("m,n,k", [
+    (1, 1, 1), (63, 65, 15), (64, 64, 16), (65, 129, 17),   # 64 x 64 tiles
+    (1000, 1910, 33), (1023, 2049, 40),                     # 240 wide tiles: 64 x 64; 272: 64 x 128
+    (2049, 1025, 18)])
+def test_plain_gemm_tile_forms(gpu, ngw_ctx, m, n, k):
+    import torch
+
+    g = torch.Generator(device="cuda").manual_seed(m)
+    a = torch.randn(k, m, generator=g, device="cuda", dtype=torch.float64)   # column-major (m, k)
+    b = torch.randn(n, k, generator=g, device="cuda", dtype=torch.float64)
+    c = torch.full((n, m), float("nan"), device="cuda", dtype=torch.float64)
+    torch.cuda.synchronize()
+    ngw_ctx.gemm_f64_dev(m, n, k, a.data_ptr(), m, b.data_ptr(), k, c.data_ptr(), m)
+    ngw_ctx.synchronize()
+    ref = b.cpu().numpy() @ a.cpu().numpy()
+    assert rel_err(c.cpu().numpy(), ref) < TOL
