@@ -905,7 +905,7 @@ void k3v2_kernel(const LpOp* ops, LpOp op1, const LpStage* st, LpStage st1,
                         const int rl = rl0 + RS * (k0 + k);
                         return m0 + (rl < 16 ? 16 * q + rl : BM / 2 + 16 * q + rl - 16);
                     };
-                    auto pair = [&](int k) { return v + min(row(k), op.nc - 1) * nv; };
+                    auto pair = [&](int k) { return v + (long)min(row(k), op.nc - 1) * nv; };
 #pragma unroll
                     for (int k = 0; k < EB; ++k) {
                         sc[k] = sigc[min(row(k), op.nc - 1)];
@@ -959,7 +959,8 @@ void k3v2_kernel(const LpOp* ops, LpOp op1, const LpStage* st, LpStage st1,
                     const int c = m0 + (rl < 16 ? 16 * q + rl : BM / 2 + 16 * q + rl - 16), j0 = n0 + 4 * cg;
                     ok[g] = c < op.nc && j0 < N;
                     const int cc = min(c, op.nc - 1), jc = min(j0, N - 4);  // loads past the end re-read the last
-                    const int b = jc / nv, idx = jc - b * nv + cc * nv;
+                    const int b = jc / nv;
+                    const long idx = jc - b * nv + (long)cc * nv;
                     ii[g] = idx + (long)b * op.ld;
                     sc[g] = sigc[cc];
                     if constexpr (KIND == LP_F16) ws[g] = gload<f32x4>(op.wsc + jc);
