@@ -522,8 +522,20 @@ struct PoissonParity {
             }
         }
         const size_t percol = sizeof(double) * 8 * (size_t)(p.z.m + 1) * p.npair;
-        // the intermediate of a batch: up to 512 MiB
-        cols = (int)std::max<size_t>(1, std::min<size_t>({(size_t)n_intp, (size_t)(512L << 20) / percol, 4096}));
+        // Columns of a batch: all where 512 MiB hold their intermediate, else
+        // whole rounds of the forward and inverse grids (one workgroup per plane
+        // and column) over the 256 CUs.  With two and more planes per CU the
+        // intermediate then stays within the 256 MiB cache between the kernels;
+        // with one, few rounds fit that, and 512 MiB are faster.  114^3 (512
+        // resident planes, 29 a column), 2000 columns: 34.2 - 34.7 ms for batches
+        // of 34 and 35, 37.6 for 36, 36.0 for the 77 of 512 MiB; 158^3 (256 planes,
+        // 40 a column), 600 columns: 29.8 ms for 12, 28.5 for 32; a 60^3 box's 400
+        // columns 1.36 ms in one batch, 1.39 in two.
+        const int percu = std::max<int>(1, std::min<int>(4, (int)((160 << 10) / lds)));  // 512 threads each
+        const size_t most = (size_t)(512L << 20) / percol, fit = percu > 1 ? most / 2 : most;
+        const size_t planes = (size_t)p.z.m + 1, round = 256 * (size_t)percu;
+        const size_t whole = fit * planes / round * round / planes;
+        cols = (int)std::max<size_t>(1, std::min<size_t>({(size_t)n_intp, 4096, (size_t)n_intp <= most ? most : whole ? whole : fit}));
         NGW_TRY(map.ensure(sizeof(int) * hmap.size()));
         NGW_TRY(vw.ensure(sizeof(double) * (size_t)hp * p.npair));
         NGW_TRY(b.ensure(percol * cols));

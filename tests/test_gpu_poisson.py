@@ -91,3 +91,17 @@ def test_coincident_grid_points_go_to_the_fft(ngw_ctx):
     zeta[np.all(g == 0, axis=1)] = zeta[-1]
     got = ngw_ctx.isdf_coulomb_kernel(zeta, g, (24, 24, 24), 0.5, 5.0)
     assert rel_err(got, O.isdf_kernel(zeta, g, (24, 24, 24), 0.5, 5.0)) < TOL
+
+
+@pytest.mark.parametrize("extent,nfft,n_intp,head", [
+    ((28, 28, 28), (114, 114, 114), 120, 20),   # batches of 35, 35, 35 and 15 columns
+    ((28, 28, 28), (114, 114, 114), 77, 20),    # the last size of one batch
+    ((39, 39, 39), (158, 158, 158), 35, 10),    # 32 and 3
+])
+def test_coulomb_kernel_batches(ngw_ctx, extent, nfft, n_intp, head):
+    """Columns of the first and the last batch against calls of their own."""
+    grid, zeta = _case(extent, nfft, n_intp, n_intp)
+    m = ngw_ctx.isdf_coulomb_kernel(zeta, grid, nfft, 0.4, 7.5)
+    for cols in (slice(0, head), slice(n_intp - head, n_intp)):
+        part = ngw_ctx.isdf_coulomb_kernel(np.asfortranarray(zeta[:, cols]), grid, nfft, 0.4, 7.5)
+        assert rel_err(m[cols, cols], part) < TOL
