@@ -271,8 +271,9 @@ int ngw_polyfit_sqrt(double xmin, double xmax, int npoly, int nx, int chebyshev,
  *   grid(3, ngrid)         integer grid coordinates in [-nfft/2, nfft/2)
  *   nfft[3]                FFT box; h grid step; trunc = R_c
  *   mmtrx(ld_m, n_intp)    output
- * Batched R2C/C2R FFTs (hipFFT) with hand-written gather / kernel-multiply /
- * scatter kernels and an FP64 MFMA GEMM for zeta^T (V zeta).
+ * Dense real transforms of the eight parity classes on FP64 MFMA (batched
+ * R2C/C2R hipFFT for supports past 47 points from the centre and boxes past
+ * 254), and an FP64 MFMA GEMM for zeta^T (V zeta).
  */
 int ngw_isdf_coulomb_kernel(ngw_context* ctx, int ngrid, int n_intp, const double* zeta,
                             long ld_zeta, const int* grid, const int* nfft, double h,
