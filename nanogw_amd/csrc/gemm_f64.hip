@@ -21,7 +21,7 @@
 
 namespace ngw {
 
-static int tiles(long m, int bm, long n, int bn) { return (int)((m + bm - 1) / bm * ((n + bn - 1) / bn)); }
+static long tiles(long m, int bm, long n, int bn) { return (m + bm - 1) / bm * ((n + bn - 1) / bn); }
 
 // ---------------------------------------------------------------- plain GEMMs
 template <int BM, int BN, class AL, class BL>
@@ -841,6 +841,10 @@ constexpr int WIDE_K3_TILES = 256;
 constexpr int DIRECT_K2_WAVES = 1024;  // 16 x 16 tiles: at most one per SIMD
 constexpr int WIDE_K2_TILES = 2048;    // 32 x 32 tiles
 constexpr int WIDE_K1_NC = 1024;
+// The runtime refuses a launch of 2^32 threads and more (64-row K1 tiles: 4096
+// points and 131,072 vectors of 128 valence states); the 128-row tiles, half as
+// many, take such a call.
+constexpr long MAX_GRID_THREADS = (1L << 32) - 1;
 
 static bool k1_direct(int nmu, int nv, int B) { return tiles(nmu, 64, (long)nv * B, 64) <= DIRECT_K1_TILES; }
 
@@ -865,7 +869,7 @@ static int launch_k1(ngw_context* ctx, const double* x, long ldx, const double* 
         };
         if (direct && tiles(nmu, 64, N, 64) <= DIRECT_K1_TILES / 4) go(k1_direct_kernel<1, 2>, 16);
         else if (direct) go(k1_direct_kernel<2, 2>, 32);
-        else if (nc < WIDE_K1_NC) go(k1_f64_kernel<64>, 64);
+        else if (nc < WIDE_K1_NC && tiles(nmu, 64, N, K1N) * GNT <= MAX_GRID_THREADS) go(k1_f64_kernel<64>, 64);
         else go(k1_f64_kernel<128>, 128);
         NGW_HIP(hipGetLastError());
     }

@@ -1,0 +1,29 @@
+"""Dispatch rules of the operator kernels at the sizes where they change over."""
+import numpy as np
+import pytest
+
+from conftest import rel_err
+from nanogw_amd.lanczos import IsdfContext
+from test_gpu_f64_tiles import TOL, _operator, _system
+
+pytestmark = pytest.mark.gpu
+
+
+def test_more_columns_than_a_grid_of_narrow_tiles(gpu):
+    """K1 over more 64 x 64 tiles than one launch has threads for (2^32):
+    4096 points and 131,075 vectors of 128 valence states."""
+    import torch
+
+    nmu, nv, nc, b = 4096, 128, 1, 131075
+    psi, m, e = _system(nmu, nv, nc, 5)
+    x = torch.randn(b, nv * nc, device="cuda", dtype=torch.float64, generator=torch.Generator(device="cuda").manual_seed(1))
+    y = torch.full_like(x, float("nan"))
+    torch.cuda.synchronize()
+    with IsdfContext(0) as ctx:   # 22 GB of work arrays, freed with it
+        ctx.set_isdf(psi, m, e, nv)
+        ctx.matvec_dev(x.data_ptr(), y.data_ptr(), nv * nc, b)
+        ctx.synchronize()
+    assert not torch.isnan(y).any()
+    pick = np.r_[0:4, 65534:65540, b - 4:b]
+    ref = _operator(psi, m, e, nv, np.ascontiguousarray(x[pick].cpu().numpy().T), False)
+    assert rel_err(y[pick].cpu().numpy().T, ref) < TOL
