@@ -841,9 +841,9 @@ constexpr int WIDE_K3_TILES = 256;
 constexpr int DIRECT_K2_WAVES = 1024;  // 16 x 16 tiles: at most one per SIMD
 constexpr int WIDE_K2_TILES = 2048;    // 32 x 32 tiles
 constexpr int WIDE_K1_NC = 1024;
-// The runtime refuses a launch of 2^32 threads and more (64-row K1 tiles: 4096
-// points and 131,072 vectors of 128 valence states); the 128-row tiles, half as
-// many, take such a call.
+// A launch counts its threads in 32 bits and runs only the remainder of a larger
+// one, without an error (64-row K1 tiles: 4096 points and 131,072 vectors of 128
+// valence states): the 128-row tiles, half as many, take such a call.
 constexpr long MAX_GRID_THREADS = (1L << 32) - 1;
 
 static bool k1_direct(int nmu, int nv, int B) { return tiles(nmu, 64, (long)nv * B, 64) <= DIRECT_K1_TILES; }
