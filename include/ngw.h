@@ -344,11 +344,14 @@ int ngw_gemm_f64_dev(ngw_context* ctx, int m, int n, int k, const double* d_a, l
  * keeps the fastest of each for later calls on this context (and batches
  * created from it) and returns the chosen indices.  A no-op in FP64 mode.
  * ngw_set_tile_config sets the indices (0 .. NGW_NTILE_CONFIGS - 1)
- * directly; index 0 is the default.
+ * directly.  While none were tuned or set, index 0 is taken, in FP16 for
+ * launches of many tiles a wider one that gives the same bits;
+ * ngw_get_tile_config returns the indices that a call over nvec vectors takes.
  */
 #define NGW_NTILE_CONFIGS 6
 int ngw_autotune(ngw_context* ctx, int nvec, int reps, int* k1_cfg, int* k3_cfg);
 int ngw_set_tile_config(ngw_context* ctx, int k1_cfg, int k3_cfg);
+int ngw_get_tile_config(ngw_context* ctx, int nvec, int* k1_cfg, int* k3_cfg);
 
 /*
  * Per-launch kernel timing with HIP events on the context's stream (no

@@ -385,6 +385,7 @@ int ngw_autotune(ngw_context* ctx, int nvec, int reps, int* k1_cfg, int* k3_cfg)
     a.x = x.as<double>(); a.ldx = ctx->ncv; a.nvec = nvec; a.out = y.as<double>(); a.ldo = ctx->ncv;
     double best1 = 1e300, best3 = 1e300;
     int b1 = 0, b3 = 0, st = NGW_OK;
+    const int old1 = ctx->lp_cfg[prec][0], old3 = ctx->lp_cfg[prec][1];
     for (int c = 0; c < NGW_NTILE_CONFIGS && st == NGW_OK; ++c) {
         ctx->lp_cfg[prec][0] = c;
         ctx->lp_cfg[prec][1] = c;
@@ -396,8 +397,8 @@ int ngw_autotune(ngw_context* ctx, int nvec, int reps, int* k1_cfg, int* k3_cfg)
         if (ctx->prof_ms[KC_K1] < best1) { best1 = ctx->prof_ms[KC_K1]; b1 = c; }
         if (ctx->prof_ms[KC_K3] < best3) { best3 = ctx->prof_ms[KC_K3]; b3 = c; }
     }
-    ctx->lp_cfg[prec][0] = b1;
-    ctx->lp_cfg[prec][1] = b3;
+    ctx->lp_cfg[prec][0] = st == NGW_OK ? b1 : old1;
+    ctx->lp_cfg[prec][1] = st == NGW_OK ? b3 : old3;
     std::copy(keep_ms, keep_ms + KC_COUNT, ctx->prof_ms);
     std::copy(keep_cnt, keep_cnt + KC_COUNT, ctx->prof_cnt);
     ctx->prof_on = was_on;
@@ -417,6 +418,14 @@ int ngw_set_tile_config(ngw_context* ctx, int k1_cfg, int k3_cfg)
     ctx->lp_cfg[ctx->precision][0] = k1_cfg;
     ctx->lp_cfg[ctx->precision][1] = k3_cfg;
     return NGW_OK;
+}
+
+int ngw_get_tile_config(ngw_context* ctx, int nvec, int* k1_cfg, int* k3_cfg)
+{
+    NGW_TRY(check_factored(ctx));
+    if (nvec <= 0 || !k1_cfg || !k3_cfg) return fail(NGW_ERR_ARG, "need nvec > 0 and two indices");
+    *k1_cfg = *k3_cfg = 0;
+    return ctx->precision == PREC_F64 ? NGW_OK : lp2_tiles(ctx, nvec, *k1_cfg, *k3_cfg);
 }
 
 int ngw_matvec_isdf_block(ngw_context* ctx, const double* vec, double* hvec, int ncv, int blksz,

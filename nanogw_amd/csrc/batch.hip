@@ -437,7 +437,7 @@ int rebuild_group(ngw_batch* b)
                 lstages[(size_t)i * npoly + sgi] = LpStage{p.x, p.out, p.y, p.alpha, p.bx, p.by, p.gamma,
                                                            p.accumulate ? 2 : 0, p.flags};
             }
-            rule.add(d);
+            rule.add(d.nmu, d.nv, d.nc, d.nvec, d.ldc1, d.ldm1);
         }
         P(NTAB_AB, i + 1) = P(NTAB_AB, i) + B;
     }

@@ -53,9 +53,8 @@ constexpr int L2K2 = 64;
 // (M-group x mod PM) x (N-group x / PM): with PM > 1 each XCD touches only its
 // share of the A operand, which then stays in that XCD's L2, while the tiles
 // of one N column (M fastest inside the rectangle) share their B slab.  Index
-// 0 is the default (for large FP16 launches it stands for a wider tile with the
-// same results, see LpTileRule::pick); the autotuner (ngw_autotune) times all of
-// them on the caller's shape.
+// 0 is the default, but for large FP16 launches (LpTileRule::pick); the
+// autotuner (ngw_autotune) times all of them on the caller's shape.
 struct LpCfg {
     int bm, bn, d, pm;
     int fw = 0;  // K3 only: 1 = W formed in the slab loader (no wprep pass)
@@ -1176,8 +1175,8 @@ void lp2_fill(const ngw_context* op, int kind, int nvec, long ld, int tda, char*
     d.q = nullptr; d.w = nullptr; d.a = nullptr; d.b = nullptr; d.niter = 0; d.kstep = nullptr;
 }
 
-// Tiles of a launch whose configuration index is 0: 128 x 256 for FP16 launches
-// of two such tiles per CU and more, if k is deep enough for the longer
+// Tiles of a launch for which none were chosen: index 0, but 128 x 256 for FP16
+// launches of two such tiles per CU and more, if k is deep enough for the longer
 // epilogue and the LDS of the third buffer to pay: fewer bytes through LDS and
 // L2 per MFMA.  Measured us, 128 x 128 and 128 x 256, K1 / K3 at Nmu, Nv, Nc and
 // vectors: (5000, 100, 1500) 1200: 2265 -> 2008 / 2847 -> 2425, 128: 254 -> 232 /
@@ -1185,19 +1184,30 @@ void lp2_fill(const ngw_context* op, int kind, int nvec, long ld, int tda, char*
 // 153 (157), K1's k = 448 / 232 -> 209; (444, 37, 370) 1200: 44 (45) / 103 (124).
 constexpr int BIG_TILES = 512, BIG_K = 1024;
 static_assert(K1_CFG[2][4].bn == 256 && K3_CFG[2][5].bn == 256, "FP16 configurations for large launches");
-void LpTileRule::add(const LpOp& d)
+void LpTileRule::add(int nmu, int nv, int nc, int nvec, int ldc1, int ldm1)
 {
-    const long nt = ((long)d.nv * d.nvec + 255) / 256;
-    tiles1 += (d.nmu + 127) / 128 * nt;
-    tiles3 += (d.nc + 127) / 128 * nt;
-    k1 = std::min(k1, d.ldc1);
-    k3 = std::min(k3, d.ldm1);
+    const long nt = ((long)nv * nvec + 255) / 256;
+    tiles1 += (nmu + 127) / 128 * nt;
+    tiles3 += (nc + 127) / 128 * nt;
+    k1 = std::min(k1, ldc1);
+    k3 = std::min(k3, ldm1);
 }
 void LpTileRule::pick(int kind, int& c1, int& c3) const
 {
-    if (kind != PREC_F16) return;
-    if (c1 == 0 && tiles1 >= BIG_TILES && k1 >= BIG_K) c1 = 4;
-    if (c3 == 0 && tiles3 >= BIG_TILES && k3 >= BIG_K) c3 = 5;
+    const bool wide = kind == PREC_F16;
+    if (c1 < 0) c1 = wide && tiles1 >= BIG_TILES && k1 >= BIG_K ? 4 : 0;
+    if (c3 < 0) c3 = wide && tiles3 >= BIG_TILES && k3 >= BIG_K ? 5 : 0;
+}
+
+int lp2_tiles(ngw_context* ctx, int nvec, int& c1, int& c3)
+{
+    NGW_TRY(lp2_prepare(ctx));
+    c1 = ctx->lp_cfg[ctx->precision][0];
+    c3 = ctx->lp_cfg[ctx->precision][1];
+    LpTileRule rule;
+    rule.add(ctx->n_intp, ctx->nval, ctx->ncond, nvec, ctx->ldc1, ctx->ldm1);
+    rule.pick(ctx->precision, c1, c3);
+    return NGW_OK;
 }
 
 void lp2_grid_counts(int kind, int c1, int c3, const LpOp& d, int* tot)
@@ -1223,10 +1233,8 @@ int operator_lp2(ngw_context* ctx, const OperatorArgs& a)
         return fail(NGW_ERR_ARG, "low-precision operator needs one leading dimension and acc == out");
     d.q = const_cast<double*>(a.v0);
     LpStage st{a.x, a.out, a.y, a.alpha, a.bx, a.by, a.v0 ? a.gamma : 0.0, a.acc ? 1 : 0, a.flags};
-    int c1 = ctx->lp_cfg[kind][0], c3 = ctx->lp_cfg[kind][1];
-    LpTileRule rule;
-    rule.add(d);
-    rule.pick(kind, c1, c3);
+    int c1, c3;
+    NGW_TRY(lp2_tiles(ctx, B, c1, c3));
     int tot[LP_NKERNEL];
     lp2_grid_counts(kind, c1, c3, d, tot);
     const int* pre[LP_NKERNEL] = {};

@@ -92,8 +92,9 @@ struct ngw_context {
     bool lp2_ready = false;
     int ldc1 = 0, ldm1 = 0;
     ngw::DevBuf pct32, pc32, pctb, pcb, pcth, pch, m32t, psiv32, psiv_scale, xsig, dpairs, lpwork;
-    // chosen {K1, K3} tile configuration per precision mode (ngw_autotune)
-    int lp_cfg[ngw::PREC_COUNT][2] = {};
+    // chosen {K1, K3} tile configuration per precision mode (ngw_autotune,
+    // ngw_set_tile_config); -1 until one is chosen: by the launch's size
+    int lp_cfg[ngw::PREC_COUNT][2] = {{-1, -1}, {-1, -1}, {-1, -1}, {-1, -1}, {-1, -1}};
     // explicit pair matrix C (n_intp x ncv, ngw_set_explicit_c) in place of
     // the factored Psi_v o Psi_c, and the workspaces of the explicit and
     // one-vector products (scaled input, partial sums of split sums)

@@ -203,13 +203,15 @@ void lp2_fill(const ngw_context* op, int kind, int nvec, long ld, int tda, char*
 // xprep, K1, slot reduction, K2, wprep, K3): the number of workgroup prefix
 // tables a grouped launch needs.
 constexpr int LP_NKERNEL = 7;
-// Default tiles of a launch over one or more requests.
+// Tiles of a launch over one or more requests where none were chosen (index -1).
 struct LpTileRule {
     long tiles1 = 0, tiles3 = 0;  // 128 x 256 tiles of K1 and K3
     int k1 = 1 << 30, k3 = 1 << 30;  // shortest k
-    void add(const LpOp& d);
+    void add(int nmu, int nv, int nc, int nvec, int ldc1, int ldm1);
     void pick(int kind, int& c1, int& c3) const;
 };
+// tile configurations of a launch over nvec vectors of the context's operator
+int lp2_tiles(ngw_context* ctx, int nvec, int& c1, int& c3);
 void lp2_grid_counts(int kind, int c1, int c3, const LpOp& d, int* tot);
 int operator_lp2(ngw_context* ctx, const OperatorArgs& a);
 

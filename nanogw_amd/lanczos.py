@@ -317,6 +317,12 @@ class IsdfContext:
     def set_tile_config(self, k1, k3):
         _lib.check(self._lib.ngw_set_tile_config(self._h, int(k1), int(k3)), "ngw_set_tile_config")
 
+    def tile_config(self, nvec):
+        """(k1_index, k3_index) that a call over nvec vectors takes."""
+        a, b = C.c_int(), C.c_int()
+        _lib.check(self._lib.ngw_get_tile_config(self._h, int(nvec), C.byref(a), C.byref(b)), "ngw_get_tile_config")
+        return a.value, b.value
+
     # ------------------------------------------------------------ profiling
     KERNEL_CLASSES = ("K1", "K2", "K3", "lanczos_ab", "cfrac", "pvectors", "sigma", "convert")
 

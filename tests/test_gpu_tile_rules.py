@@ -9,6 +9,24 @@ from test_gpu_f64_tiles import TOL, _operator, _system
 pytestmark = pytest.mark.gpu
 
 
+def test_a_chosen_tile_configuration_is_used_as_given(gpu):
+    """Every index names one tile at every launch width; only while none was
+    set or tuned does the size decide."""
+    nmu, nv, nc, wide = 1100, 33, 1030, 500   # 9 x 65 tiles of 128 x 256 in K1 and K3, k 1056 and 1120
+    with IsdfContext(0) as ctx:
+        ctx.set_isdf(*_system(nmu, nv, nc, 3), nv)
+        assert ctx.tile_config(wide) == (0, 0)   # FP64
+        for prec in ("f32", "bf16", "bf16x3", "f16"):
+            ctx.set_precision(prec)
+            assert ctx.tile_config(9) == (0, 0)
+            assert ctx.tile_config(wide) == ((4, 5) if prec == "f16" else (0, 0))
+            chosen = ctx.autotune(wide, reps=1)
+            assert ctx.tile_config(wide) == ctx.tile_config(9) == chosen
+            for c in range(6):
+                ctx.set_tile_config(c, 5 - c)
+                assert ctx.tile_config(wide) == ctx.tile_config(9) == (c, 5 - c)
+
+
 def test_more_columns_than_a_grid_of_narrow_tiles(gpu):
     """K1 over more 64 x 64 tiles than one launch has threads for (2^32):
     4096 points and 131,075 vectors of 128 valence states."""
