@@ -880,7 +880,7 @@ void k3v2_kernel(const LpOp* ops, LpOp op1, const LpStage* st, LpStage st1,
                 // step) and has EB elements' loads in flight: consecutive
                 // lanes read consecutive pairs of one c
                 constexpr int RS = GNT / BN > 0 ? GNT / BN : 1, EB = ROOM ? 8 : 4;
-                static_assert(EPR / RS % EB == 0, "epilogue element batches");
+                static_assert(EPR / RS % EB == 0 && 16 % (EB * RS) == 0, "epilogue element batches");
                 const int col = (int)threadIdx.x % BN, j = n0 + col;
                 if ((int)threadIdx.x >= RS * BN || j >= N) return;
                 const int b = j / nv, v = j - b * nv, rl0 = (int)threadIdx.x / BN;
@@ -905,6 +905,7 @@ void k3v2_kernel(const LpOp* ops, LpOp op1, const LpStage* st, LpStage st1,
                         return m0 + (rl < 16 ? 16 * q + rl : BM / 2 + 16 * q + rl - 16);
                     };
                     auto pair = [&](int k) { return v + (long)min(row(k), op.nc - 1) * nv; };
+                    if (row(0) >= op.nc) continue;  // none of the batch's rows (see skip below)
 #pragma unroll
                     for (int k = 0; k < EB; ++k) {
                         sc[k] = sigc[min(row(k), op.nc - 1)];
@@ -950,13 +951,23 @@ void k3v2_kernel(const LpOp* ops, LpOp op1, const LpStage* st, LpStage st1,
                 o4 ar[GU];
                 long ii[GU];
                 float sc[GU];
-                bool ok[GU];
+                bool ok[GU], skip = true;
+                int cr[GU], jr[GU];
 #pragma unroll
                 for (int g = 0; g < GU; ++g) {
                     const int e = threadIdx.x + GNT * (k0 + g);
                     const int rl = e / G, cg = e - rl * G;
-                    const int c = m0 + (rl < 16 ? 16 * q + rl : BM / 2 + 16 * q + rl - 16), j0 = n0 + 4 * cg;
-                    ok[g] = c < op.nc && j0 < N;
+                    cr[g] = m0 + (rl < 16 ? 16 * q + rl : BM / 2 + 16 * q + rl - 16);
+                    jr[g] = n0 + 4 * cg;
+                    ok[g] = cr[g] < op.nc && jr[g] < N;
+                    skip = skip && !ok[g];
+                }
+                // a small operator's tile is mostly past the end: 20 of 128
+                // rows at nc = 20, where reading the rest took K3 from 15 to 19 us
+                if (skip) continue;
+#pragma unroll
+                for (int g = 0; g < GU; ++g) {
+                    const int c = cr[g], j0 = jr[g];
                     const int cc = min(c, op.nc - 1), jc = min(j0, N - 4);  // loads past the end re-read the last
                     const int b = jc / nv;
                     const long idx = jc - b * nv + (long)cc * nv;

@@ -5,6 +5,7 @@ import pytest
 from conftest import rel_err
 from nanogw_amd.lanczos import IsdfContext
 from test_gpu_f64_tiles import TOL, _operator, _system
+from test_gpu_lowp_tiles import TOL as LOWP_TOL
 
 pytestmark = pytest.mark.gpu
 
@@ -45,3 +46,24 @@ def test_more_columns_than_a_grid_of_narrow_tiles(gpu):
     pick = np.r_[0:4, 65534:65540, b - 4:b]
     ref = _operator(psi, m, e, nv, np.ascontiguousarray(x[pick].cpu().numpy().T), False)
     assert rel_err(y[pick].cpu().numpy().T, ref) < TOL
+
+
+@pytest.mark.parametrize("prec", ["f32", "bf16", "bf16x3", "f16"])
+@pytest.mark.parametrize("nv", [3, 4])   # K3's element-wise and 16-byte epilogues
+@pytest.mark.parametrize("nc", [1, 8, 15, 16, 17, 63, 65, 72, 80, 129])
+def test_k3_tiles_mostly_past_the_end(ngw_ctx, prec, nv, nc):
+    """K3 tiles of 128 rows with all but a few past nc: what the epilogue
+    skips and what it writes meet at every group and batch of rows."""
+    nmu, b = 60, 23
+    psi, m, e = _system(nmu, nv, nc, nc)
+    m *= nmu
+    x = np.random.default_rng(nv).normal(size=(nv * nc, b))
+    ngw_ctx.set_isdf(psi, m, e, nv)
+    ngw_ctx.set_precision(prec)
+    try:
+        y = ngw_ctx.matvec_isdf_BLOCK(x, tamm_d=True)
+    finally:
+        ngw_ctx.set_precision("f64")
+    d = ((e[nv:, None] - e[None, :nv]).reshape(-1))[:, None] * x
+    ref = _operator(psi, m, e, nv, x, True) - d
+    assert np.abs(y - d - ref).max() < LOWP_TOL[prec] * np.abs(ref).max()
