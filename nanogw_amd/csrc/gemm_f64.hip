@@ -112,10 +112,13 @@ int gemm_f64_tn(hipStream_t s, int m, int n, int k, double alpha, const double* 
 // tiles, two or three per CU, and k is the grid: without the ranges the CUs
 // with three set the time (10.5 ms for k = 97,000, now 8.3; the full product on 128 x
 // 128 tiles 11.4).  Range partials lie tile after tile; sym_sum_kernel adds
-// them in order and writes each element and its mirror.
+// them in order and writes each element and its mirror.  With one range (4033
+// columns and more, or k below 4096) the tile is written as it is: partials
+// would take half of C's size again.
 constexpr int SYM = 64;
+template <bool SPLIT>
 __global__ __launch_bounds__(GNT) void gemm_sym_kernel(ColMajorAT al, ColMajorB bl, int k, int kc, int ntiles,
-                                                       double* part)
+                                                       double* part, int n, double alpha, double* c, long ldc)
 {
     __shared__ SmemF64<SYM, SYM> sm;
     const int id = xcd_tile(blockIdx.x, gridDim.x), split = id / ntiles, tile = id - split * ntiles;
@@ -127,9 +130,19 @@ __global__ __launch_bounds__(GNT) void gemm_sym_kernel(ColMajorAT al, ColMajorB 
     al.a += k0;
     bl.b += k0;
     AccF64<SYM, SYM> acc;
-    gemm_f64_tile<SYM, SYM>(al, bl, (tile - tn * (tn + 1) / 2) * SYM, tn * SYM, min(kc, k - (int)k0), acc, sm);
-    double* o = part + (long)id * SYM * SYM;
-    for_acc_f64<SYM, SYM>(acc, [&](int row, int col, double val) { o[row + col * SYM] = val; });
+    const int m0 = (tile - tn * (tn + 1) / 2) * SYM, n0 = tn * SYM;
+    gemm_f64_tile<SYM, SYM>(al, bl, m0, n0, min(kc, k - (int)k0), acc, sm);
+    if constexpr (SPLIT) {
+        double* o = part + (long)id * SYM * SYM;
+        for_acc_f64<SYM, SYM>(acc, [&](int row, int col, double val) { o[row + col * SYM] = val; });
+    } else {
+        for_acc_f64<SYM, SYM>(acc, [&](int row, int col, double val) {
+            const int gm = m0 + row, gn = n0 + col;
+            if (gm >= n || gn >= n) return;
+            c[gm + (long)gn * ldc] = alpha * val;
+            if (m0 != n0) c[gn + (long)gm * ldc] = alpha * val;
+        });
+    }
 }
 
 __global__ __launch_bounds__(256) void sym_sum_kernel(const double* part, int S, int ntiles, int n, double alpha,
@@ -160,9 +173,17 @@ int gemm_f64_tn_sym(hipStream_t s, int n, int k, double alpha, const double* a, 
     int S = std::max(1, std::min((2048 + ntiles - 1) / ntiles, k / 2048));
     const int kc = (k + S - 1) / S;
     S = (k + kc - 1) / kc;
+    const ColMajorAT al{a, lda, n};
+    const ColMajorB bl{b, ldb, n};
+    if (S == 1) {
+        hipLaunchKernelGGL(gemm_sym_kernel<false>, dim3(ntiles), dim3(GNT), 0, s, al, bl, k, kc, ntiles, nullptr, n,
+                           alpha, c, ldc);
+        NGW_HIP(hipGetLastError());
+        return NGW_OK;
+    }
     NGW_TRY(part.ensure(sizeof(double) * (size_t)S * ntiles * SYM * SYM));
-    hipLaunchKernelGGL(gemm_sym_kernel, dim3(ntiles * S), dim3(GNT), 0, s, ColMajorAT{a, lda, n}, ColMajorB{b, ldb, n},
-                       k, kc, ntiles, part.as<double>());
+    hipLaunchKernelGGL(gemm_sym_kernel<true>, dim3(ntiles * S), dim3(GNT), 0, s, al, bl, k, kc, ntiles,
+                       part.as<double>(), n, alpha, c, ldc);
     hipLaunchKernelGGL(sym_sum_kernel, dim3(ntiles), dim3(256), 0, s, part.as<const double>(), S, ntiles, n, alpha, c,
                        ldc);
     NGW_HIP(hipGetLastError());

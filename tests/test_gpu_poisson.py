@@ -105,3 +105,40 @@ def test_coulomb_kernel_batches(ngw_ctx, extent, nfft, n_intp, head):
     for cols in (slice(0, head), slice(n_intp - head, n_intp)):
         part = ngw_ctx.isdf_coulomb_kernel(np.asfortranarray(zeta[:, cols]), grid, nfft, 0.4, 7.5)
         assert rel_err(m[cols, cols], part) < TOL
+
+
+def test_coulomb_kernel_memory_of_many_columns(gpu, ngw_ctx):
+    """12,000 columns: M on the device, V zeta, zeta and the transforms'
+    intermediate, and no second array of M's order (half of M would be 0.6
+    GB); M against the oracle on the first, last and middle columns."""
+    import threading
+
+    import torch
+
+    from oracle import oracle as O
+
+    n = 12000
+    g, zeta = _case((4, 4, 4), (10, 10, 10), n, 7)
+    ngw_ctx.isdf_coulomb_kernel(zeta[:, :64], g, (10, 10, 10), 0.4, 2.0)   # code objects loaded
+    free = [torch.cuda.mem_get_info(0)[0]]
+    done = threading.Event()
+
+    def watch():
+        while not done.wait(0.002):
+            free.append(torch.cuda.mem_get_info(0)[0])
+
+    t = threading.Thread(target=watch)
+    t.start()
+    try:
+        m = ngw_ctx.isdf_coulomb_kernel(zeta, g, (10, 10, 10), 0.4, 2.0)
+    finally:
+        done.set()
+        t.join()
+    pick = np.r_[0:3, 6000:6003, n - 3:n]
+    ref = O.isdf_kernel(np.asfortranarray(zeta[:, pick]), g, (10, 10, 10), 0.4, 2.0)
+    assert rel_err(m[np.ix_(pick, pick)], ref) < TOL
+    assert np.array_equal(m[:64, 64:], m[64:, :64].T)
+    inter = 8 * 8 * 5 * 6 * 32 * min(n, 4096)                # 8 classes x (m + 1) x h x 32 frequencies a column
+    need = 8 * (n * n + 2 * n * len(g)) + inter
+    print("used", free[0] - min(free), "need", need)
+    assert free[0] - min(free) < need + (128 << 20)
