@@ -927,7 +927,7 @@ static int launch_k3(ngw_context* ctx, const double* u, int B, const OperatorEpi
         const int mt = (nc + bm - 1) / bm, n = mt * (int)((N + bn - 1) / bn);
         hipLaunchKernelGGL(kernel, dim3(n), dim3(nt), 0, ctx->stream, al, bl, nmu, nc, nv, B, ep, mt, n);
     };
-    const int t64 = tiles(nc, 64, N, 64);
+    const long t64 = tiles(nc, 64, N, 64);
     if (t64 <= DIRECT_K3_TILES) {
         if (tiles(nc, 16, N, 16) <= 1024) go(k3_direct_kernel<1, 1, 4>, 16, 16, 64);
         else go(k3_direct_kernel<2, 1, 4>, 32, 16, 64);

@@ -67,3 +67,59 @@ def test_k3_tiles_mostly_past_the_end(ngw_ctx, prec, nv, nc):
     d = ((e[nv:, None] - e[None, :nv]).reshape(-1))[:, None] * x
     ref = _operator(psi, m, e, nv, x, True) - d
     assert np.abs(y - d - ref).max() < LOWP_TOL[prec] * np.abs(ref).max()
+
+
+@pytest.mark.parametrize("nmu,nc,nv,blksz,tiles", [
+    (1100, 1030, 33, 500, (4, 5)),   # 9 x 65 tiles of 128 x 256 in K1 and K3, remainders in M and N
+    (1100, 1030, 32, 520, (4, 5)),   # K3's 16-byte epilogue
+    (1100, 700, 20, 1100, (0, 5)),   # k of K1 704; 6 x 86 tiles in K3, 16-byte epilogue
+    (900, 1281, 129, 130, (4, 0)),   # 8 x 66 tiles in K1, vectors of two partial sums; k of K3 960
+    (600, 1030, 300, 90, (4, 0)),    # 5 x 106 tiles in K1, vectors of three and four partial sums
+    (1100, 1030, 33, 400, (0, 0)),   # 9 x 52
+])
+def test_wide_fp16_tiles_keep_the_bits_of_the_narrow_ones(gpu, nmu, nc, nv, blksz, tiles):
+    """The tiles the size rule takes for large FP16 launches, against the
+    128 x 128 ones on the same call and on its first columns alone (a column's
+    place decides where K1's partial sums are cut, so only leading columns keep
+    their bits)."""
+    psi, m, e = _system(nmu, nv, nc, nmu + nc)
+    m *= nmu
+    x = np.random.default_rng(blksz).normal(size=(nv * nc, blksz))
+    with IsdfContext(0) as ctx:
+        ctx.set_isdf(psi, m, e, nv)
+        ctx.set_precision("f16")
+        assert ctx.tile_config(blksz) == tiles
+        assert ctx.tile_config(9) == (0, 0)
+        wide = ctx.matvec_isdf_BLOCK(x)
+        few = ctx.matvec_isdf_BLOCK(x[:, :9])
+        ctx.set_tile_config(0, 0)
+        assert ctx.tile_config(blksz) == (0, 0)
+        narrow = ctx.matvec_isdf_BLOCK(x)
+    assert np.array_equal(wide, narrow)
+    assert np.array_equal(wide[:, :9], few)
+    d = ((e[nv:, None] - e[None, :nv]).reshape(-1) ** 2)[:, None] * x[:, -6:]
+    ref = _operator(psi, m, e, nv, x[:, -6:], False) - d
+    assert np.abs(wide[:, -6:] - d - ref).max() < LOWP_TOL["f16"] * np.abs(ref).max()
+
+
+@pytest.mark.parametrize("nmu,nv,nc,blksz", [
+    (401, 25, 37, 700),    # 26 x 44 K2 tiles of 16 x 16, more than a wave per SIMD: 13 x 22 of 32 x 32
+    (515, 1, 20, 601),     # 33 x 38, and K1 without LDS: K2 adds the two slots of a vector
+    (515, 2, 70, 299),     # 33 x 19 = 627: 16 x 16 waves, adding the slots
+    (2048, 1, 18, 1025),   # 64 x 33 = 2112 tiles of 32 x 32: 128 x 64
+])
+def test_f64_k2_forms(ngw_ctx, nmu, nv, nc, blksz):
+    """K2's 32 x 32 LDS tiles and the sizes beside them.  Leading columns have
+    the same bits in calls of every width from two on; one vector alone takes
+    kernels that split its sums, and agrees to rounding."""
+    psi, m, e = _system(nmu, nv, nc, nmu)
+    x = np.random.default_rng(nmu).normal(size=(nv * nc, blksz))
+    ngw_ctx.set_isdf(psi, m, e, nv)
+    ngw_ctx.set_precision("f64")
+    y = ngw_ctx.matvec_isdf_BLOCK(x)
+    pick = np.r_[0:20, blksz // 2:blksz // 2 + 20, blksz - 20:blksz]
+    assert rel_err(y[:, pick], _operator(psi, m, e, nv, x[:, pick], False)) < TOL
+    for n in (2, 35, 261):
+        assert np.array_equal(ngw_ctx.matvec_isdf_BLOCK(x[:, :n]), y[:, :n]), n
+    one = ngw_ctx.matvec_isdf_BLOCK(x[:, :1])
+    assert rel_err(one, y[:, :1]) < TOL
