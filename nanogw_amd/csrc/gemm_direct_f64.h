@@ -3,10 +3,10 @@
 // from global memory into a ring of D register sets, D - 1 blocks of 16 k
 // ahead of the block being multiplied.
 //
-// For products whose 64 x 128 LDS tiles would leave most of the 1024 SIMDs
-// idle: a 16 x 16 tile per wave gives 32 times as many waves, and the ring
-// covers the memory latency that a lone wave per SIMD cannot hide behind
-// others.  The k order of every sum is that of gemm_core_f64.h (blocks of 16,
+// For products whose LDS tiles would leave most of the 1024 SIMDs idle: a
+// 16 x 16 tile per wave gives four times as many waves as 64 x 64 tiles on four
+// waves, eight times as many as 128 x 64, and the ring covers the memory
+// latency that a lone wave per SIMD cannot hide behind others.  The k order of every sum is that of gemm_core_f64.h (blocks of 16,
 // sub-step s of lane group g takes k = 4 g + s), so both cores give the same
 // bits.
 //

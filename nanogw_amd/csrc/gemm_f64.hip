@@ -13,8 +13,10 @@
 // (lanczos_spectra_BLOCK.F90:91-95).
 //
 // K1's reduction over v writes per-tile partial sums to a slot buffer instead
-// of using atomics; a small kernel sums the slots in a fixed order, so every
-// result is bitwise independent of how many other vectors share the launch.
+// of using atomics; a small kernel sums the slots in a fixed order.  A column's
+// bits depend on its place in the call (where its slots are cut), not on how
+// many columns follow, for calls of two and more; one column alone takes
+// operator_f64_one, which splits the sums.
 
 #include "gemm_direct_f64.h"
 #include "operator_loaders.h"
@@ -52,7 +54,7 @@ static int gemm_plain(hipStream_t s, const AL& al, const BL& bl, int m, int n, i
         hipLaunchKernelGGL(kernel, dim3(mt * nt), dim3(GNT), 0, s, al, bl, m, n, k, alpha, c, ldc, mt, mt * nt);
     };
     if (m <= 0 || n <= 0) return NGW_OK;
-    if (tiles(m, 64, n, 128) < 256) go(gemm_plain_kernel<64, 64, AL, BL>, 64);
+    if (tiles(m, 64, n, 128) < NCU) go(gemm_plain_kernel<64, 64, AL, BL>, 64);
     else go(gemm_plain_kernel<64, 128, AL, BL>, 128);
     NGW_HIP(hipGetLastError());
     return NGW_OK;
@@ -170,7 +172,7 @@ int gemm_f64_tn_sym(hipStream_t s, int n, int k, double alpha, const double* a, 
     if (n <= 0) return NGW_OK;
     const int nt = (n + SYM - 1) / SYM, ntiles = nt * (nt + 1) / 2;
     // about eight workgroups per CU, ranges of at least 2048
-    int S = std::max(1, std::min((2048 + ntiles - 1) / ntiles, k / 2048));
+    int S = std::max(1, std::min((8 * NCU + ntiles - 1) / ntiles, k / 2048));
     const int kc = (k + S - 1) / S;
     S = (k + kc - 1) / kc;
     const ColMajorAT al{a, lda, n};
@@ -773,13 +775,16 @@ int operator_f64_one(ngw_context* ctx, const OperatorArgs& a)
     // against 17.8 and 20.8 with two); the largest molecules take 64-row K1
     // tiles and two per CU (5000 x 100 x 1500: K1 57 us against 65 - 81 for the
     // other choices, K3 51 against 66 with one; 3000 x 64 x 700: 27 us
-    // against 20 with the 32-row tiles).
+    // against 20 with the 32-row tiles).  Whole calls, large form / small form:
+    // 3000 x 70 x 800 77 / 65 us, 3600 x 72 x 900 92 / 78, 4200 x 90 x 900
+    // 99 / 101, 4000 x 100 x 1000 105 / 93, 4500 x 100 x 1200 124 / 139,
+    // 5000 x 100 x 1500 145 / 184: they meet at 3.4e8 to 5e8, above the line.
     const bool big = nv > 32 && nmu > 1 && (double)nmu * nv * nc >= OV_BIG;
     const int fn1 = nv <= 16 || nmu < 2 ? 1 : nv <= 32 ? 2 : 4, nch1 = (nv + 16 * fn1 - 1) / (16 * fn1);
     const int nch3 = (nv + 63) / 64, fn3 = ((nv + nch3 - 1) / nch3 + 15) / 16;
     const int bm1 = big ? 2 * OVM : OVM;
     const int mt1 = (nmu + bm1 - 1) / bm1, mt3 = (nc + OVM - 1) / OVM;
-    const int want = big ? 512 : 256;
+    const int want = big ? 2 * NCU : NCU;
     int S1 = ov_splits(mt1 * nch1, nc, want), S3 = ov_splits(mt3 * nch3, nmu, want);
     const int kc = (nc + S1 - 1) / S1, kmu = (nmu + S3 - 1) / S3;
     S1 = (nc + kc - 1) / kc;
@@ -848,19 +853,24 @@ int operator_f64_one(ngw_context* ctx, const OperatorArgs& a)
 // 0.2 us, so few tiles go to the small forms; with every CU busy the larger
 // tiles win through fewer loads per MFMA.  Measured (us, nmu x nv x nc, B):
 //   K1 480x8x56, 8: 7 direct / 11.6 64x64; 731x13x129, 37: 12.4 / 15.9;
-//      1000x24x250, 80: 40 / 33; 2000x40x400, 800: 1062 64x64 / 1149 128x64;
-//      5000x100x1500, 200: 5665 / 5507
+//      1000x24x250, 80: 40 / 33; 1000x24x250, 100: 42 64x64 / 51 128x64;
+//      2000x40x400, 40: 77 / 73; 2000x40x400, 800: 1064 / 1056;
+//      5000x100x1500, 4: 195 / 233; 5000x100x1500, 100: 2914 / 2848
+//      (128 rows are 0 to 5% faster once both forms fill their rounds of
+//      workgroups, and up to 17% slower where a few tiles more than a round are
+//      left for the last one: that, not nc, is what parts the two, and the line
+//      at nc = 1024 only keeps the largest operators on 128 rows)
 //   K2 480, 256: 10 direct / 14 32x32 / 22 64x64; 5000, 40: 98 / 124 / 168;
 //      2000, 200: 79 / 54 / 74; 5000, 200: 450 / 247 / 333;
 //      5000, 1600: 1661 32x32 / 1278 128x64
 //   K3 480x8x56, 256: 16 direct / 28 64x64 / 44 128x64; 1000x24x250, 80:
 //      42 / 51 / 82; 2000x40x400, 40: 134 / 89 / 139; 2000x40x400, 200:
 //      500 / 281 / 258; 5000x100x1500, 200: 5241 64x64 / 4575 128x64
-constexpr int DIRECT_K1_TILES = 256;  // 64 x 64 tiles: at most one per CU
-constexpr int DIRECT_K3_TILES = 128;
-constexpr int WIDE_K3_TILES = 256;
-constexpr int DIRECT_K2_WAVES = 1024;  // 16 x 16 tiles: at most one per SIMD
-constexpr int WIDE_K2_TILES = 2048;    // 32 x 32 tiles
+constexpr int DIRECT_K1_TILES = NCU;  // 64 x 64 tiles: at most one per CU
+constexpr int DIRECT_K3_TILES = NCU / 2;
+constexpr int WIDE_K3_TILES = NCU;
+constexpr int DIRECT_K2_WAVES = 4 * NCU;  // 16 x 16 tiles: at most one per SIMD
+constexpr int WIDE_K2_TILES = 8 * NCU;    // 32 x 32 tiles
 constexpr int WIDE_K1_NC = 1024;
 // A launch counts its threads in 32 bits and runs only the remainder of a larger
 // one, without an error (64-row K1 tiles: 4096 points and 131,072 vectors of 128
@@ -929,7 +939,7 @@ static int launch_k3(ngw_context* ctx, const double* u, int B, const OperatorEpi
     };
     const long t64 = tiles(nc, 64, N, 64);
     if (t64 <= DIRECT_K3_TILES) {
-        if (tiles(nc, 16, N, 16) <= 1024) go(k3_direct_kernel<1, 1, 4>, 16, 16, 64);
+        if (tiles(nc, 16, N, 16) <= 4 * NCU) go(k3_direct_kernel<1, 1, 4>, 16, 16, 64);
         else go(k3_direct_kernel<2, 1, 4>, 32, 16, 64);
     } else if (t64 <= WIDE_K3_TILES) {
         go(k3_f64_kernel<64, 64>, 64, 64, GNT);

@@ -1193,7 +1193,7 @@ void lp2_fill(const ngw_context* op, int kind, int nvec, long ld, int tda, char*
 // vectors: (5000, 100, 1500) 1200: 2265 -> 2008 / 2847 -> 2425, 128: 254 -> 232 /
 // 336 -> 332, 48 (760 / 228 tiles): 101 -> 92 / 137 (181); (2000, 40, 400) 1200:
 // 153 (157), K1's k = 448 / 232 -> 209; (444, 37, 370) 1200: 44 (45) / 103 (124).
-constexpr int BIG_TILES = 512, BIG_K = 1024;
+constexpr int BIG_TILES = 2 * NCU, BIG_K = 1024;
 static_assert(K1_CFG[2][4].bn == 256 && K3_CFG[2][5].bn == 256, "FP16 configurations for large launches");
 void LpTileRule::add(int nmu, int nv, int nc, int nvec, int ldc1, int ldm1)
 {

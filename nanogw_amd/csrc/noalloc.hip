@@ -13,9 +13,10 @@ namespace ngw {
 
 namespace {
 
-// qp_newton_kernel's work arrays: 5 nen doubles per QP state (x, f, Im f and
-// the two spline vectors).  Every entry a call reads is written earlier in
-// the same call, so nothing has to be cleared between calls.
+// qp_newton_kernel's work arrays: 5 nen doubles per QP state, of which tables
+// too long for LDS use 3 nen (the table and the two spline vectors).  Every
+// entry a call reads is written earlier in the same call, so nothing has to be
+// cleared between calls.
 constexpr long QP_SCRATCH_DOUBLES = 5L * NGW_QP_NOALLOC_MAX_POINTS;
 static __device__ __align__(256) double scratch[QP_SCRATCH_DOUBLES];
 

@@ -129,7 +129,7 @@ __global__ void coulomb_kernel(int n1, int n2, int n3, double h, double trunc, d
 //   pt_forward  fold one pair of planes z = +-az, transform x and y
 //   pt_kernel   transform z, multiply, transform z back (in place)
 //   pt_inverse  transform y and x back, unfold to the grid points
-// The intermediate is 8 (m + 1) h^2 doubles per column (6.9 MB at 114^3).
+// The intermediate is 8 (m + 1) h x 16 HT doubles per column (6.9 MB at 114^3).
 // Measured on 2000 columns of a 114^3 box (97,000 points): 24 ms against
 // 270 ms of batched hipFFT D2Z / Z2D (Bluestein transforms for 114 = 2 3 19).
 // Every matrix is padded with zeros to the kernels' 16 MT positions by 16 HT
@@ -533,7 +533,7 @@ struct PoissonParity {
         // columns 1.36 ms in one batch, 1.39 in two.
         const int percu = std::max<int>(1, std::min<int>(4, (int)((160 << 10) / lds)));  // 512 threads each
         const size_t most = (size_t)(512L << 20) / percol, fit = percu > 1 ? most / 2 : most;
-        const size_t planes = (size_t)p.z.m + 1, round = 256 * (size_t)percu;
+        const size_t planes = (size_t)p.z.m + 1, round = NCU * (size_t)percu;
         const size_t whole = fit * planes / round * round / planes;
         cols = (int)std::max<size_t>(1, std::min<size_t>({(size_t)n_intp, 4096, (size_t)n_intp <= most ? most : whole ? whole : fit}));
         NGW_TRY(map.ensure(sizeof(int) * hmap.size()));
